@@ -18,10 +18,9 @@ __device__ __forceinline__ float ordkey_inv(uint32_t k) {
 // CAP: the most candidates a row can have (its vocabulary size)
 template <int CAP>
 struct SampleSmemT {
-  unsigned long long cand[CAP];
+  __align__(16) unsigned long long cand[CAP];
   float w[CAP];
   unsigned int hist[256];
-  float red[ST / 64];
   int nkeep;
   int ncand;  // candidates placed so far
   int code;  // the drawn code, for the waves that build the next level's input
@@ -144,31 +143,43 @@ __device__ float radix_kth(const float (&x)[NE], int V, int k, SM& sm) {
   return ordkey_inv(pre);
 }
 
-// After this returns, sm.cand[0 .. sm.nkeep) holds the kept candidates in sampling order and sm.w their weights.
-// x[] holds this thread's elements i = tid + 256*e (e < NE, NE * 256 >= V) of the transformed row.
-template <int NE, class SM>
-__device__ void topk_select(const float (&x)[NE], int V, int k, SM& sm) {
-  const int tid = threadIdx.x;
-  const float NEG = -INFINITY;
-  sm.hist[tid] = 0;  // ordered before the histograms by the max's barrier
-  unsigned int* h2 = reinterpret_cast<unsigned int*>(sm.cand);  // the coarse histogram (candidates come later)
-  h2[tid] = 0;
-  if (tid == 0) {
-    sm.nkeep = 0;
-    sm.ncand = 0;
+// The k-th largest of 256 values held 4 a lane by every wave, approximately: a value t with at least k of them >= t,
+// at most k + k / 16 unless values repeat or crowd within the search's reach. lo: a value with count(>= lo) >= k.
+// Three thresholds a round (their counts are independent, a round is bound by the latency of one): 4-5 rounds.
+__device__ __forceinline__ float wave_kth(const float (&c)[4], float lo, float hi, int k) {
+  const int enough = k + (k >> 4);
+  for (int it = 0; it < 12; ++it) {
+    const float m2 = 0.5f * lo + 0.5f * hi;
+    const float m1 = 0.5f * lo + 0.5f * m2, m3 = 0.5f * m2 + 0.5f * hi;
+    if (!(m2 > lo && m2 < hi)) break;
+    int n1 = 0, n2 = 0, n3 = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      n1 += __popcll(__ballot(c[i] >= m1));
+      n2 += __popcll(__ballot(c[i] >= m2));
+      n3 += __popcll(__ballot(c[i] >= m3));
+    }
+    // counts fall from lo to hi: the highest threshold that still has k
+    int n = 0;
+    if (n3 >= k) lo = m3, n = n3;
+    else if (n2 >= k) lo = m2, hi = m3, n = n2;
+    else if (n1 >= k) lo = m1, hi = m2, n = n1;
+    else hi = m1;
+    if (n && n <= enough) break;
   }
-  float lm = NEG;
-#pragma unroll
-  for (int e = 0; e < NE; ++e)
-    if (tid + ST * e < V) lm = fmaxf(lm, x[e]);
-  // row max: wave maxima meet in LDS behind one barrier (sm.red is next written by a later call, after further
-  // barriers)
-  lm = wave_max_dpp(lm);
-  if ((tid & 63) == 0) sm.red[tid >> 6] = lm;
+  return lo;
+}
+
+// The candidate marks (bit e: element e) of a row with a large k (more than KFAST): bucket counts of floor(32 * (m - x)).
+template <int NE, class SM>
+__device__ bool hist_marks(const float (&x)[NE], int V, int k, float m, SM& sm, unsigned int& mark) {
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  unsigned int* h2 = reinterpret_cast<unsigned int*>(sm.cand);  // the coarse histogram (candidates come later)
+  __syncthreads();  // every wave has read the threads' maxima
+  sm.hist[tid] = 0;
+  h2[tid] = 0;
   __syncthreads();
-  float m = sm.red[0];
-#pragma unroll
-  for (int i = 1; i < ST / 64; ++i) m = fmaxf(m, sm.red[i]);
   int bk[NE];
 #pragma unroll
   for (int e = 0; e < NE; ++e) {
@@ -182,27 +193,22 @@ __device__ void topk_select(const float (&x)[NE], int V, int k, SM& sm) {
   __syncthreads();
   // every wave finds b* itself from the histogram (no barrier): lane l holds bins 4 l .. 4 l + 3; bin 255 (8 or
   // more below the max) is not counted
-  int bstar;
-  unsigned int near = 0;  // elements within 8 of the max, when fewer than k
-  {
-    const int lane = tid & 63;
-    unsigned int c[4];
+  unsigned int c[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) c[i] = 4 * lane + i < 255 ? sm.hist[4 * lane + i] : 0u;
-    int idx;
-    unsigned int before;
-    wave_find_bin(c, (unsigned int)k, idx, before);
-    bstar = idx < 0 ? 255 : idx;
-    if (idx < 0) near = (unsigned int)__builtin_amdgcn_readlane((int)wave_incl_scan(c[0] + c[1] + c[2] + c[3]), 63);
-  }
-  // Fewer than k elements within 8 of the max (a peaked row, the usual case for a confident model): a coarse
-  // histogram of the rest, 0.5 wide bins from 255/32 below the max (bin 255: 135 or more below, not counted), finds
-  // the bin b2 where the count reaches k; the candidates are then the near elements and those in coarse bins <= b2.
+  for (int i = 0; i < 4; ++i) c[i] = 4 * lane + i < 255 ? sm.hist[4 * lane + i] : 0u;
+  int bstar;
+  unsigned int before;
+  wave_find_bin(c, (unsigned int)k, bstar, before);
+  // Fewer than k elements within 8 of the max: a coarse histogram of the rest, 0.5 wide bins from 255/32 below the
+  // max (bin 255: 135 or more below, not counted), finds the bin b2 where the count reaches k; the candidates are
+  // then the near elements and those in coarse bins <= b2.
   int b2 = 0;
   int cb[NE];
 #pragma unroll
   for (int e = 0; e < NE; ++e) cb[e] = 255;
-  if (bstar == 255) {
+  if (bstar < 0) {
+    const unsigned int near =
+        (unsigned int)__builtin_amdgcn_readlane((int)wave_incl_scan(c[0] + c[1] + c[2] + c[3]), 63);
 #pragma unroll
     for (int e = 0; e < NE; ++e) {
       if (tid + ST * e < V && bk[e] == 255) {
@@ -212,70 +218,156 @@ __device__ void topk_select(const float (&x)[NE], int V, int k, SM& sm) {
       }
     }
     __syncthreads();
-    const int lane = tid & 63;
-    unsigned int c[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) c[i] = 4 * lane + i < 255 ? h2[4 * lane + i] : 0u;
-    unsigned int before;
     wave_find_bin(c, (unsigned int)k - near, b2, before);
     __syncthreads();  // every wave's scan of the coarse histogram precedes the candidate stores over it
+    if (b2 < 0) return false;
   }
+  mark = 0;
+#pragma unroll
+  for (int e = 0; e < NE; ++e)
+    mark |= (tid + ST * e < V && (bstar >= 0 ? bk[e] <= bstar : (bk[e] < 255 || cb[e] <= b2))) ? 1u << e : 0u;
+  return true;
+}
 
-  // Fewer than k elements within 135 of the max (or -inf / NaN among the top k): the candidates are the elements
-  // >= the exact k-th largest (all elements when no valid one exists), found by radix select, rather than the
-  // whole row, so the rank placement below still applies.
-  const bool radix = bstar == 255 && b2 < 0;
-  const float kth_sel = radix ? radix_kth<NE>(x, V, k, sm) : 0.f;
-  const bool all = kth_sel != kth_sel;
-  // compaction: one LDS atomic per wave reserves the wave's places (their order does not matter: the candidates
-  // are ranked by key below); lanes take consecutive places by ballot rank
+// After this returns, sm.cand[0 .. sm.nkeep) holds the kept candidates in sampling order and sm.w their weights.
+// x[] holds this thread's elements i = tid + 256*e (e < NE, NE * 256 >= V) of the transformed row.
+//
+// Candidates (any set {x >= t} with t at or below the k-th largest gives the same kept set): for k <= KFAST, t is
+// about the k-th largest of the 256 threads' maxima, found by every wave by bisection over the values. At least k
+// elements, the maxima themselves, are then >= t, and a random order of the row leaves few others: 55 candidates for
+// k = 50 of 2048. It needs no atomics and one barrier, whatever the shape of the row; a histogram of the distances below
+// the maximum serialised its atomics on a peaked row, whose bulk falls into a few bins. Rows of 2048 with one code 16
+// above the bulk, MI355X: the 224-seat depth frame (30 such samplers) 5.11 -> 4.94 ms, the one-seat frame 2.35 ->
+// 2.21 ms; head and codebook-0 sampler of 224 flat rows 24.2 -> 21.4 us. Larger k takes the histogram: the maxima would
+// let through several times k candidates (k = 200 of 2048: about 350). More than 256 candidates (an order that gathers
+// the leaders in a few threads, many repeats), or fewer than k threads with a maximum above -inf, take the exact radix
+// select.
+// The kernel runs every line of code once or twice a launch, so it is bound by latencies (dependent operations, barriers,
+// instruction fetch) and short loops beat unrolled code.
+constexpr int KFAST = 128;
+
+template <int NE, class SM>
+__device__ void topk_select(const float (&x)[NE], int V, int k, SM& sm) {
+  const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const unsigned long long below = (1ull << lane) - 1ull;
-  unsigned long long masks[NE];
-  int total = 0;
-#pragma unroll
-  for (int e = 0; e < NE; ++e) {
-    const bool near_e = bstar < 255 ? bk[e] <= bstar : (bk[e] < 255 || cb[e] <= b2);
-    masks[e] = __ballot(tid + ST * e < V && (radix ? (all || x[e] >= kth_sel) : near_e));
-    total += __popcll(masks[e]);
+  const float NEG = -INFINITY;
+  if (tid == 0) {
+    sm.nkeep = 0;
+    sm.ncand = 0;
   }
-  int base = 0;
-  if (lane == 0 && total > 0) base = (int)atomicAdd((unsigned int*)&sm.ncand, (unsigned int)total);
-  base = __builtin_amdgcn_readfirstlane(base);
+  if (tid < 128) sm.cand[tid] = 0ull;  // below every candidate's key
+  float lm = NEG;
 #pragma unroll
-  for (int e = 0; e < NE; ++e) {
-    const int i = tid + ST * e;
-    if ((masks[e] >> lane) & 1ull)
-      sm.cand[base + __popcll(masks[e] & below)] =
-          ((unsigned long long)ordkey(x[e]) << 32) | (unsigned long long)(0xffffffffu - (uint32_t)i);
-    base += __popcll(masks[e]);
-  }
+  for (int e = 0; e < NE; ++e)
+    if (tid + ST * e < V) lm = fmaxf(lm, x[e]);
+  sm.hist[tid] = __float_as_uint(lm);
   __syncthreads();
-  const int nc = sm.ncand;
+  float c[4];
+  int valid = 0;
+  float hi = NEG, lo = INFINITY;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    c[i] = __uint_as_float(sm.hist[4 * lane + i]);
+    valid += __popcll(__ballot(c[i] > NEG));
+    hi = fmaxf(hi, c[i]);
+    lo = fminf(lo, c[i] > NEG ? c[i] : INFINITY);
+  }
+  hi = wave_max_dpp(hi);
+  bool exact = false, all = false;  // exact: t is the k-th largest itself
+  float t = NEG;
+  unsigned int hmark = 0;
+  bool have = false;  // the histogram's marks
+  if (k > KFAST) {
+    have = hist_marks<NE>(x, V, k, hi, sm, hmark);
+    exact = !have;
+  } else if (valid >= k) {
+    t = wave_kth(c, -wave_max_dpp(-lo), hi, k);
+  } else {
+    exact = true;
+    __syncthreads();  // every wave has read the maxima; sm.cand is free
+  }
+  int nc;
+  for (;;) {
+    if (exact) {
+      t = radix_kth<NE>(x, V, k, sm);
+      all = t != t;  // no valid element
+    }
+    if (exact || have) {  // histograms lay over the candidates
+      if (tid < 128) sm.cand[tid] = 0ull;
+      __syncthreads();
+    }
+    // compaction: every lane marks its candidates; one LDS atomic per wave reserves the wave's places (their order
+    // does not matter: the candidates are ranked by key below), and each round stores a lane's lowest remaining mark,
+    // in ballot order. Two or three rounds: a lane rarely holds more, and the loop's few lines of code are fetched
+    // once where a store per element was fetched NE times.
+    unsigned int mark = 0;
+    if (!have) {
+#pragma unroll
+      for (int e = 0; e < NE; ++e) mark |= (tid + ST * e < V && (all || x[e] >= t)) ? 1u << e : 0u;
+    } else {
+      mark = hmark;
+    }
+    const unsigned int mine = __popc(mark);
+    const unsigned int upto = wave_incl_scan(mine);
+    const int total = __builtin_amdgcn_readlane((int)upto, 63);
+    int base = 0;
+    if (lane == 0 && total > 0) base = (int)atomicAdd((unsigned int*)&sm.ncand, (unsigned int)total);
+    int at = __builtin_amdgcn_readfirstlane(base) + (int)(upto - mine);
+    while (__ballot(mark != 0)) {
+      const int e = __ffs((int)mark) - 1;
+      float v = x[0];
+#pragma unroll
+      for (int q = 1; q < NE; ++q) v = e == q ? x[q] : v;
+      if (mark != 0)
+        sm.cand[at++] = ((unsigned long long)ordkey(v) << 32) | (unsigned long long)(0xffffffffu - (uint32_t)(tid + ST * e));
+      mark &= mark - 1;
+    }
+    __syncthreads();
+    nc = sm.ncand;
+    if (have || exact || nc <= ST) break;
+    __syncthreads();  // every wave has read the count
+    if (tid == 0) sm.ncand = 0;  // ordered before the next compaction by the radix select's barriers
+    exact = true;
+  }
   int P2 = 2;
   while (P2 < nc) P2 <<= 1;
-  if (nc <= 64) {
+  if (nc <= 128) {
     // The usual case: rank placement with the count split over the waves. Keys are distinct (the index is part
-    // of the key), so candidate l goes to position #{j : key_j > key_l}; wave w counts the keys j in
-    // [16 w, 16 w + 16) (LDS broadcast reads), the four partial counts meet in sm.hist (free by now).
-    const unsigned long long key = lane < nc ? sm.cand[lane] : 0ull;
-    const int j0 = 16 * wave;
-    int part = 0;
-    if (j0 < nc) {
-      unsigned long long c16[16];
+    // of the key), so candidate l goes to position #{j : key_j > key_l}. A lane takes candidates lane and lane + 64;
+    // wave w counts the keys j in [J w, J w + J) (LDS broadcast reads), J = 16 or 32; the partial counts of both
+    // (packed in 16 bits each) meet in sm.hist (free by now).
+    const unsigned long long key0 = sm.cand[lane];  // 0 past the last candidate, up to 128
+    const unsigned long long key1 = sm.cand[64 + lane];
+    unsigned int part = 0;
+    auto count16 = [&](int j0, bool two) {
+      if (j0 >= nc) return;
+      ulonglong2 c2[8];
 #pragma unroll
-      for (int q = 0; q < 16; ++q) c16[q] = sm.cand[min(j0 + q, nc - 1)];
+      for (int q = 0; q < 8; ++q) c2[q] = *reinterpret_cast<const ulonglong2*>(&sm.cand[j0 + 2 * q]);
 #pragma unroll
-      for (int q = 0; q < 16; ++q) part += (j0 + q < nc && c16[q] > key) ? 1 : 0;
+      for (int q = 0; q < 8; ++q) {
+        part += (c2[q].x > key0 ? 1u : 0u) + (c2[q].y > key0 ? 1u : 0u);
+        if (two) part += (c2[q].x > key1 ? 0x10000u : 0u) + (c2[q].y > key1 ? 0x10000u : 0u);
+      }
+    };
+    if (nc <= 64) {
+      count16(16 * wave, false);
+    } else {
+      count16(32 * wave, true);
+      count16(32 * wave + 16, true);
     }
-    sm.hist[tid] = (unsigned int)part;
+    sm.hist[tid] = part;
     __syncthreads();
-    if (tid < nc) sm.cand[sm.hist[lane] + sm.hist[64 + lane] + sm.hist[128 + lane] + sm.hist[192 + lane]] = key;
+    if (tid < nc) {
+      const unsigned int r = sm.hist[lane] + sm.hist[64 + lane] + sm.hist[128 + lane] + sm.hist[192 + lane];
+      sm.cand[tid < 64 ? r & 0xffffu : r >> 16] = tid < 64 ? key0 : key1;
+    }
     __syncthreads();
   } else if (nc <= ST) {
-    // The usual case (top-k of a peaked row): rank placement. Keys are distinct (the index is part of the key),
-    // so candidate t goes to position #{j : key_j > key_t}; the reads of key_j are LDS broadcasts.
+    // rank placement, one candidate a thread; the reads of key_j are LDS broadcasts
     const unsigned long long key = tid < nc ? sm.cand[tid] : 0ull;
     int rank = 0;
     if ((tid & ~63) < nc) {  // waves holding no candidate skip the count
@@ -295,8 +387,8 @@ __device__ void topk_select(const float (&x)[NE], int V, int k, SM& sm) {
   __syncthreads();
   for (int kk = 2; kk <= P2; kk <<= 1) {
     for (int j = kk >> 1; j > 0; j >>= 1) {
-      for (int t = tid; t < (P2 >> 1); t += ST) {
-        const int i = ((t & ~(j - 1)) << 1) | (t & (j - 1));
+      for (int t2 = tid; t2 < (P2 >> 1); t2 += ST) {
+        const int i = ((t2 & ~(j - 1)) << 1) | (t2 & (j - 1));
         const int p = i | j;
         const unsigned long long a = sm.cand[i], b = sm.cand[p];
         const bool desc = (i & kk) == 0;
@@ -329,88 +421,106 @@ __device__ __forceinline__ float lanef(float v, int q) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), q));
 }
 
-// Running sums of the weights of cand[0..n) in order, skipping index `skip` (-1: none), by one wave: the weights of
-// 64 candidates sit one per lane (a skipped or absent one as +0.0) and are broadcast in order through readlane;
-// lane j adds weight q through fmaf(w_q, f, c) with f = 1 for q <= j and 0 after, so it holds exactly the
-// sequential fp32 sum w_0 + ... + w_j (fmaf(w, 1, c) rounds c + w once; fmaf(w, 0, c) = c), and lane 63 holds
-// the chunk's total, carried into the next chunk. No lane-dependent select is needed, so the chain is 64
-// independent-operand fmas. Running sums of chunks after the first are stored over their weights in sm.w.
-// Returns the total (same value in every lane); *last = position of the last term, -1 if none; *first_use /
-// *first_run = the first chunk's ballot of terms and this lane's running sum.
-template <class SM>
-__device__ float wave_prefix(SM& sm, int n, int skip, int* last, unsigned long long* first_use, float* first_run) {
-  const int lane = threadIdx.x & 63;
-  const float lf = (float)lane;
-  float carry = 0.f;
-  int l = -1;
-  for (int j0 = 0; j0 < n; j0 += 64) {
-    const int j = j0 + lane;
-    const bool in = j < n && cand_index(sm.cand[j]) != skip;
-    const float wsel = in ? sm.w[j] : 0.f;
-    const unsigned long long use = __ballot(in);
-    float c = carry;
-#pragma unroll
-    for (int q = 0; q < 64; ++q)
-      c = fmaf(lanef(wsel, q), __builtin_amdgcn_fmed3f(lf - (float)q + 1.0f, 0.0f, 1.0f), c);
-    carry = lanef(c, 63);
-    if (use) l = j0 + 63 - __clzll((long long)use);
-    if (j0 == 0) {
-      *first_use = use;
-      *first_run = c;
-    } else if (j < n) {
-      sm.w[j] = c;
-    }
+// Sequential fp32 running sums of 64 values, 4 a lane in lanes 0..15 (w): run = carry + w_0 + ... in order, every sum
+// rounded as one running total's. A lane adds its 4 values to the total that the lane before it holds (DPP row_shr:1;
+// lane 0 reads +0 and has carry in its first value), 16 times over: lane l is final after l + 1 rounds and repeats the
+// same sums from then on. Returns the total in every lane. One lane a value took 63 cross-lane steps and twice the
+// time; rows 1..3 of the wave run along on their own values, unused.
+__device__ __forceinline__ float wave_seq_scan(float4 w, float carry, float4& run) {
+  if ((threadIdx.x & 63) == 0) w.x = carry + w.x;
+  run = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 2
+  for (int q = 0; q < 16; ++q) {
+    const float in = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(run.w), 0x111, 0xf, 0xf, true));
+    run.x = in + w.x;
+    run.y = run.x + w.y;
+    run.z = run.y + w.z;
+    run.w = run.z + w.w;
   }
-  *last = l;
-  return carry;
+  return lanef(run.w, 15);
 }
 
-// Inverse-CDF pick over cand[0..n) skipping index `skip`: the first position whose running sum (the same
-// sequential fp32 order as the total S) exceeds u * S, else the last term; -1 when the weights sum to 0.
-// Called by one whole wave; every lane returns the same index. Overwrites sm.w past the first 64 candidates.
+// The weights of positions j0 + 4 l .. + 3 of the kept set (lane l < 16; +0 past n).
+template <class SM>
+__device__ __forceinline__ float4 weights4(const SM& sm, int j0, int n) {
+  const int j = j0 + 4 * (int)(threadIdx.x & 15);
+  float4 w;
+  w.x = sm.w[min(j, n - 1)];
+  w.y = sm.w[min(j + 1, n - 1)];
+  w.z = sm.w[min(j + 2, n - 1)];
+  w.w = sm.w[min(j + 3, n - 1)];
+  if (j >= n) w.x = 0.f;
+  if (j + 1 >= n) w.y = 0.f;
+  if (j + 2 >= n) w.z = 0.f;
+  if (j + 3 >= n) w.w = 0.f;
+  return w;
+}
+
+// Lane 0..15's first of its four running sums above t, over the wave: the position within the 64, or -1.
+__device__ __forceinline__ int first_above(const float4& run, float t) {
+  const int sub = run.x > t ? 0 : run.y > t ? 1 : run.z > t ? 2 : 3;
+  const unsigned long long hit = __ballot((threadIdx.x & 63) < 16 && run.w > t);  // the sums do not fall
+  if (!hit) return -1;
+  const int l = __ffsll((long long)hit) - 1;
+  return 4 * l + __builtin_amdgcn_readlane(sub, l);
+}
+
+// Inverse-CDF pick over cand[0..n) skipping index `skip` (-1: none): the first position whose running sum (the same
+// sequential fp32 order as the total S) exceeds u * S, else the last term; -1 when the weights sum to 0. A skipped
+// position counts +0, so its running sum is the one before it and is never the first above. Called by one whole wave;
+// every lane returns the same index. Rows of more than 64 candidates sum twice. Zeroes the skipped weight in sm.w.
 template <class SM>
 __device__ int pick(SM& sm, int n, float u, int skip) {
   const int lane = threadIdx.x & 63;
-  int last;
-  unsigned long long use0 = 0;
-  float run0 = 0.f;
-  const float S = wave_prefix(sm, n, skip, &last, &use0, &run0);
+  if (n <= 0) return -1;
+  int last = n - 1;
+  if (skip >= 0) {
+    for (int j0 = 0; j0 < n; j0 += 64) {
+      const int j = j0 + lane;
+      const bool is = j < n && cand_index(sm.cand[j]) == skip;
+      if (is) sm.w[j] = 0.f;
+    }
+    __builtin_amdgcn_wave_barrier();
+    if (cand_index(sm.cand[last]) == skip) --last;
+  }
+  float4 run;
+  float S = wave_seq_scan(weights4(sm, 0, n), 0.f, run);
+  for (int j0 = 64; j0 < n; j0 += 64) {
+    float4 r;
+    S = wave_seq_scan(weights4(sm, j0, n), S, r);
+  }
   if (last < 0 || !(S > 0.f)) return -1;
   const float t = u * S;
-  unsigned long long hit = use0 & __ballot(run0 > t);
-  if (hit) return cand_index(sm.cand[__ffsll((long long)hit) - 1]);
-  for (int j0 = 64; j0 < n; j0 += 64) {
-    const int j = j0 + lane;
-    hit = __ballot(j < n && cand_index(sm.cand[j]) != skip && sm.w[j] > t);
-    if (hit) return cand_index(sm.cand[j0 + __ffsll((long long)hit) - 1]);
+  int at = first_above(run, t);
+  if (at < 0 && n > 64) {
+    float c = lanef(run.w, 15);
+    for (int j0 = 64; j0 < n && at < 0; j0 += 64) {
+      float4 r;
+      c = wave_seq_scan(weights4(sm, j0, n), c, r);
+      at = first_above(r, t);
+      if (at >= 0) at += j0;
+    }
   }
-  return cand_index(sm.cand[last]);
+  return cand_index(sm.cand[at >= 0 && at <= last ? at : last]);
 }
 
 // Top-p cut of the kept set cand[0..n) (maya3/engine.py:669-672: a candidate is dropped when the probability mass
 // sorted before it exceeds top_p): position j stays while run_(j-1) / S <= top_p, where run is the sequential fp32
-// running sum of the weights in order (the fmaf broadcast of wave_prefix) and S their total in the same order.
+// running sum of the weights in order (wave_seq_scan) and S their total in the same order.
 // The kept set stays a prefix of the order. Called by one whole wave; leaves sm.w unchanged; returns the new
 // length (>= 1) in every lane.
 template <class SM>
 __device__ int top_p_keep(const SM& sm, int n, float top_p) {
-  const float lf = (float)(threadIdx.x & 63);
-  auto chunk_runs = [&](int j0, float carry) {
-    const int j = j0 + (int)(threadIdx.x & 63);
-    const float wj = j < n ? sm.w[j] : 0.f;
-    float c = carry;
-#pragma unroll
-    for (int q = 0; q < 64; ++q) c = fmaf(lanef(wj, q), __builtin_amdgcn_fmed3f(lf - (float)q + 1.0f, 0.0f, 1.0f), c);
-    return c;
-  };
   float S = 0.f;
-  for (int j0 = 0; j0 < n; j0 += 64) S = lanef(chunk_runs(j0, S), 63);
+  float4 r;
+  for (int j0 = 0; j0 < n; j0 += 64) S = wave_seq_scan(weights4(sm, j0, n), S, r);
   float carry = 0.f;
   for (int j0 = 0; j0 < n; j0 += 64) {
-    const float c = chunk_runs(j0, carry);  // lane l: run_(j0 + l)
-    carry = lanef(c, 63);
-    const unsigned long long cut = __ballot(j0 + (int)(threadIdx.x & 63) + 1 < n && c / S > top_p);
-    if (cut) return j0 + __ffsll((long long)cut);  // first j with run_j / S > top_p keeps 0..j
+    carry = wave_seq_scan(weights4(sm, j0, n), carry, r);
+    // the first j with run_j / S > top_p keeps 0 .. j (the quotients do not fall)
+    const float4 p = make_float4(r.x / S, r.y / S, r.z / S, r.w / S);
+    const int at = first_above(p, top_p);
+    if (at >= 0) return min(j0 + at + 1, n);
   }
   return n;
 }

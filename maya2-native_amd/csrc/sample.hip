@@ -13,12 +13,9 @@
 // This is inverse-CDF sampling of the top-k renormalised softmax, the distribution the reference draws with
 // Gumbel/exponential races (serve/fast_depth_kernels.py:60-68, maya3/engine.py:687-688).
 //
-// Selection inside one 256-thread workgroup per row: the row max m, a 256-bin histogram of the bucket
-// floor(32*(m - x)) (bin 255 = everything 8 or more below the max, not counted), the first bin b* at which the
-// cumulative count reaches k, then every x with bucket <= b* is a candidate. The bucket is monotone in x, so
-// the candidates contain the top k and all its ties. When fewer than k elements lie within 8 of the max (a peaked
-// row), a radix select over the ordered keys finds the exact k-th largest instead, and the candidates are the
-// elements >= it. Candidates are ordered by rank placement (at most 256) or a bitonic sort.
+// Selection inside one 256-thread workgroup per row (topk_select): a value t at or below the k-th largest, then every
+// x >= t is a candidate, so the candidates contain the top k and all its ties. Candidates are ordered by rank
+// placement (at most 256) or a bitonic sort.
 #include "m3x_sample.h"
 
 // ---------------------------------------------------------------------------------------------------------
@@ -219,15 +216,18 @@ __device__ __forceinline__ T slot_or(const T* p, long i, const void* dummy, T df
   return p ? v : dflt;
 }
 
+// NE: elements per thread (V <= 256 NE).
+template <int NE>
 __global__ __launch_bounds__(ST) void cb0_sample_kernel(Cb0Args a) {
   __shared__ SampleSmem sm;
   __shared__ int64_t hist[CB0_HMAX];
+  __shared__ uint32_t seen[NE * ST / 32];  // bit i: code i is in the slot's history
   const int row = blockIdx.x;
   // the logits first, every element's load issued before any is used (indices past V re-read element V - 1 and are
   // masked below: a load under a condition would make the compiler wait for it there, one round trip per element)
-  uint16_t raw[SMAXV / ST];
+  uint16_t raw[NE];
 #pragma unroll
-  for (int e = 0; e < SMAXV / ST; ++e) raw[e] = a.logits[(long)row * a.ld_l + min((int)threadIdx.x + ST * e, a.V - 1)];
+  for (int e = 0; e < NE; ++e) raw[e] = a.logits[(long)row * a.ld_l + min((int)threadIdx.x + ST * e, a.V - 1)];
   const long s = a.slots[row];
   // the slot's settings and state in one round trip
   const void* dm = a.slots + row;
@@ -241,26 +241,32 @@ __global__ __launch_bounds__(ST) void cb0_sample_kernel(Cb0Args a) {
   const int64_t frames = slot_or<int64_t>(a.frames_t, s, dm, 0), min_frames = slot_or<int64_t>(a.min_t, s, dm, 0);
   const float hz0 = slot_or(a.hazard_t, s, dm, 0.f);
   const int32_t ctr = slot_or<int32_t>(a.ctr_t, s, dm, 0);
-  const float uu = a.u[(long)row * a.ld_u];  // loaded first: its latency overlaps the selection
-  // the slot's recent codes, staged once in LDS: the repetition penalty reads them, and wave 0 writes them back
-  // shifted by one with the drawn code last
+  const float uu = a.u[(long)row * a.ld_u];  // its latency overlaps the selection
+  // the slot's recent codes, staged once in LDS: the repetition penalty marks them in a bit per code (one read per
+  // element instead of a walk over the history), and wave 0 writes them back shifted by one with the drawn code last
   const int hw = a.hist_t ? a.hist_w : 0;  // <= CB0_HMAX (checked on the host)
   const bool pen = hw > 0 && a.rep_t;
-  for (int j = threadIdx.x; j < hw; j += ST) hist[j] = a.hist_t[s * a.hist_w + j];
+  int64_t recent = -1;
+  if ((int)threadIdx.x < hw) recent = a.hist_t[s * a.hist_w + threadIdx.x];
+  if (pen) {  // uniform over the workgroup
+    if (threadIdx.x < NE * ST / 32) seen[threadIdx.x] = 0u;
+    __syncthreads();
+  }
+  if ((int)threadIdx.x < hw) {
+    hist[threadIdx.x] = recent;
+    if (pen && recent >= 0 && recent < a.V && recent != a.aeos)
+      atomicOr(&seen[(int)recent >> 5], 1u << ((int)recent & 31));
+  }
   __syncthreads();
-  float x[SMAXV / ST];
+  float x[NE];
 #pragma unroll
-  for (int e = 0; e < SMAXV / ST; ++e) {
+  for (int e = 0; e < NE; ++e) {
     const int i = threadIdx.x + ST * e;
     float v = -INFINITY;
     if (i < a.V) {
       v = bf2f(raw[e]) / temp;
       if (i == a.aeos) v = v + bias;
-      if (pen && i != a.aeos) {
-        bool seen = false;
-        for (int j = 0; j < hw; ++j) seen |= hist[j] == (int64_t)i;
-        if (seen) v = v - rep;
-      }
+      if (pen && ((seen[i >> 5] >> (i & 31)) & 1u)) v = v - rep;
     }
     x[e] = v;
   }
@@ -278,13 +284,9 @@ __global__ __launch_bounds__(ST) void cb0_sample_kernel(Cb0Args a) {
       const unsigned long long m = __ballot(j < n && cand_index(sm.cand[j]) == a.aeos);
       if (m) wa = sm.w[j0 + __ffsll((long long)m) - 1];
     }
-    float S = 0.f;  // every kept weight in order (sequential fp32), read before pick reuses sm.w
-    for (int j0 = 0; j0 < n; j0 += 64) {
-      const int j = j0 + (int)(threadIdx.x & 63);
-      const float wj = j < n ? sm.w[j] : 0.f;
-#pragma unroll
-      for (int q = 0; q < 64; ++q) S = S + lanef(wj, q);
-    }
+    float S = 0.f;  // every kept weight in order (sequential fp32), read before pick drops the AEOS weight
+    float4 run;
+    for (int j0 = 0; j0 < n; j0 += 64) S = wave_seq_scan(weights4(sm, j0, n), S, run);
     const float pa = wa / S;
     const int c = pick(sm, n, uu, a.aeos);
     const int arg = cand_index(sm.cand[0]);
@@ -324,7 +326,10 @@ M3X_API int m3x_cb0_sample(const void* logits, long ld_l, int V, int aeos, const
   Cb0Args a{(const uint16_t*)logits, ld_l, V, aeos, slots, u, ld_u, temp_t, temp, topk_t, top_k, topp_t, top_p,
             aeos_bias, rep_t,
             hist_t, hist_w, frames_t, min_t, hazard_t, ctr_t, cb0_out, cb0_i32, ld_cb0_i32, stop_out};
-  hipLaunchKernelGGL(cb0_sample_kernel, dim3(B), dim3(ST), 0, (hipStream_t)stream, a);
+  if (V <= 8 * ST)
+    hipLaunchKernelGGL((cb0_sample_kernel<8>), dim3(B), dim3(ST), 0, (hipStream_t)stream, a);
+  else
+    hipLaunchKernelGGL((cb0_sample_kernel<SMAXV / ST>), dim3(B), dim3(ST), 0, (hipStream_t)stream, a);
   M3X_CHECK_LAUNCH();
   return M3X_OK;
 }
