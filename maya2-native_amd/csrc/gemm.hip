@@ -47,11 +47,8 @@ __global__ __launch_bounds__(256) void linear_f32_kernel(const float* __restrict
   constexpr int RED = (KW - 1) * NW * NA * MT * 64 * 4;  // floats of slice partials
   __shared__ __align__(16) float xs[XS > RED ? XS : RED];
 
-  const int xcd = blockIdx.x & 7;
-  const int slot = blockIdx.x >> 3;
-  const int nb = (slot / mblk) * 8 + xcd;
-  const int mb = slot - (slot / mblk) * mblk;
-  if (nb >= nblk) return;  // padding block: the whole workgroup leaves before any barrier
+  int mb, nb;
+  if (!xcd_block(mblk, nblk, mb, nb)) return;  // padding block: the whole workgroup leaves before any barrier
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: scalar branches around the MFMAs
@@ -220,8 +217,8 @@ static bool launch_linear_f32(hipStream_t st, const float* X, long ldx, const fl
     }
   }
   const int mblk = m3x_ceil_div(M, 16 * mt), nblk = m3x_ceil_div(ntiles, nw);
-  if ((long)m3x_ceil_div(nblk, 8) * 8 * mblk > 0x7fffffffL) return false;
-  const dim3 grid(m3x_ceil_div(nblk, 8) * 8 * mblk);
+  if (xcd_grid(mblk, nblk) > 0x7fffffffL) return false;
+  const dim3 grid((unsigned)xcd_grid(mblk, nblk));
 #define M3X_LF(MTT, NWW)                                                                                     \
   hipLaunchKernelGGL((linear_f32_kernel<MTT, NWW, EPI>), grid, dim3(256), 0, st, X, ldx, W, W2, Y, ldy, M, N, K, \
                      mblk, nblk)
@@ -258,7 +255,7 @@ static int linear_common(const void* x, long ldx, const void* w, const void* w2,
     return M3X_OK;
   }
   const LinearPlan p = linear_plan(M, N, K, epi == EPI_SWIGLU, ldx);
-  if ((long)m3x_ceil_div(p.nblk, 8) * 8 * p.mblk > 0x7fffffffL) return M3X_EINVAL;
+  if (xcd_grid(p.mblk, p.nblk) > 0x7fffffffL) return M3X_EINVAL;
   hipStream_t st = (hipStream_t)stream;
   const uint16_t *X = (const uint16_t*)x, *Wt = (const uint16_t*)w, *W2 = (const uint16_t*)w2;
   uint16_t* Y = (uint16_t*)y;

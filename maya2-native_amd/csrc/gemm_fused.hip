@@ -43,7 +43,7 @@ M3X_API int m3x_linear_resid(const void* x, long ldx, const void* w_packed, cons
     return M3X_EINVAL;
   if (dtype != M3X_BF16 && dtype != M3X_F16) return M3X_EUNSUPPORTED;
   const LinearPlan p = linear_plan(M, N, K, false, ldx);
-  if ((long)m3x_ceil_div(p.nblk, 8) * 8 * p.mblk > 0x7fffffffL) return M3X_EINVAL;
+  if (xcd_grid(p.mblk, p.nblk) > 0x7fffffffL) return M3X_EINVAL;
   const ResidOut ro{(const uint16_t*)h, ldh, (const uint16_t*)c, ldc, tc, (float2*)part, norm_kind};
   hipStream_t st = (hipStream_t)stream;
   const bool ok = dtype == M3X_BF16 ? resid_launch<M3X_BF16>(p, st, x, ldx, w_packed, h_out, ld_out, M, N, K, ro)
@@ -69,7 +69,7 @@ M3X_API int m3x_linear_normed(const void* x, long ldx, const void* part, const f
     return M3X_EINVAL;
   if (dtype != M3X_BF16 && dtype != M3X_F16) return M3X_EUNSUPPORTED;
   const LinearPlan p = linear_plan(M, N, K, act == M3X_ACT_SWIGLU, ldx);
-  if ((long)m3x_ceil_div(p.nblk, 8) * 8 * p.mblk > 0x7fffffffL) return M3X_EINVAL;
+  if (xcd_grid(p.mblk, p.nblk) > 0x7fffffffL) return M3X_EINVAL;
   const NormIn ni{(const float2*)part, u, v, eps, norm_kind};
   hipStream_t st = (hipStream_t)stream;
   const bool ok = dtype == M3X_BF16
@@ -109,7 +109,7 @@ M3X_API int m3x_linear_qk_rope(const void* x, long ldx, const void* part, float 
       !aligned(wk, 16) || (part && !aligned(part, 16)))
     return M3X_EINVAL;
   const LinearPlan p = linear_plan(M, N, K, false, ldx);
-  if ((long)m3x_ceil_div(p.nblk, 8) * 8 * p.mblk > 0x7fffffffL) return M3X_EINVAL;
+  if (xcd_grid(p.mblk, p.nblk) > 0x7fffffffL) return M3X_EINVAL;
   hipStream_t st = (hipStream_t)stream;
   const NormIn ni{(const float2*)part, nullptr, nullptr, eps_in, M3X_NORM_RMS};
   const QkOut qk{(uint16_t*)q_out, s_qo_b, s_qo_h, (uint16_t*)k_cache, (uint16_t*)v_cache, sk_s, sk_h, sk_t, slots, pos,

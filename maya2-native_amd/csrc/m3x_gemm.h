@@ -17,8 +17,8 @@
 // 16*MT activation rows of each 128-wide K chunk in LDS with row-contiguous loads, double-buffered, and every
 // wave reads its fragments from there. Weight fragments run two chunks ahead in registers, activations three.
 // The KW partial sums meet in LDS and are added in slice order: the result is independent of scheduling.
-// Workgroups are numbered so that the row blocks sharing one weight slab run on one XCD (ids equal mod 8) and
-// the slab is fetched into that XCD's L2 once.
+// Workgroups are numbered so that the row blocks sharing one weight slab run on one XCD (xcd_block) and the slab is
+// fetched into that XCD's L2 once.
 //
 // Epilogues (each rounds exactly where the reference's eager ops round):
 //   EPI_NONE    y = dt(acc)
@@ -582,11 +582,8 @@ __global__ __launch_bounds__(256) void linear_kernel(const uint16_t* __restrict_
   __shared__ __align__(16) uint16_t xs[2][KW * ROWS * LDR];
   __shared__ float2 pst[PRO ? ROWS : 1];
 
-  const int xcd = blockIdx.x & 7;
-  const int slot = blockIdx.x >> 3;
-  const int nb = (slot / mblk) * 8 + xcd;
-  const int mb = slot - (slot / mblk) * mblk;
-  if (nb >= nblk) return;  // padding block: the whole workgroup leaves before any barrier
+  int mb, nb;
+  if (!xcd_block(mblk, nblk, mb, nb)) return;  // padding block: the whole workgroup leaves before any barrier
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: scalar branches
@@ -742,11 +739,8 @@ __global__ __launch_bounds__(64 * NWAVES) void linear_oneshot_kernel(const uint1
   __shared__ __align__(16) uint16_t xs[KW * ROWS * LDR];
   __shared__ float2 pst[PRO ? ROWS : 1];
 
-  const int xcd = blockIdx.x & 7;
-  const int slot = blockIdx.x >> 3;
-  const int nb = (slot / mblk) * 8 + xcd;
-  const int mb = slot - (slot / mblk) * mblk;
-  if (nb >= nblk) return;  // padding block: the whole workgroup leaves before any barrier
+  int mb, nb;
+  if (!xcd_block(mblk, nblk, mb, nb)) return;  // padding block: the whole workgroup leaves before any barrier
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: scalar branches
@@ -883,11 +877,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
   __shared__ __align__(16) uint16_t la[2][BM * LDA];
   __shared__ float2 pst[PRO ? BM : 1];
 
-  const int xcd = blockIdx.x & 7;
-  const int slot = blockIdx.x >> 3;
-  const int nb = (slot / mblk) * 8 + xcd;
-  const int mb = slot - (slot / mblk) * mblk;
-  if (nb >= nblk) return;  // padding block: the whole workgroup leaves before any barrier
+  int mb, nb;
+  if (!xcd_block(mblk, nblk, mb, nb)) return;  // padding block: the whole workgroup leaves before any barrier
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1107,11 +1098,8 @@ __global__ __launch_bounds__(256) void linear_strip_kernel(const uint16_t* __res
   uint16_t* const la0 = smem;
   uint16_t* const la1 = smem + BM * LDA;
 
-  const int xcd = blockIdx.x & 7;
-  const int slot = blockIdx.x >> 3;
-  const int nb = (slot / mblk) * 8 + xcd;
-  const int mb = slot - (slot / mblk) * mblk;
-  if (nb >= nblk) return;  // padding block: the whole workgroup leaves before any barrier
+  int mb, nb;
+  if (!xcd_block(mblk, nblk, mb, nb)) return;  // padding block: the whole workgroup leaves before any barrier
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1457,14 +1445,14 @@ static bool launch_linear(const LinearPlan& p, hipStream_t st, const uint16_t* X
                           const uint16_t* W2, uint16_t* Y, long ldy, int M, int N, int K, const NormIn& ni = NormIn{},
                           const ResidOut& ro = ResidOut{}, const QkOut& qk = QkOut{}) {
   static_assert(!(PRO && EPI == EPI_RESID), "a residual projection takes its input as is");
-  const dim3 grid(m3x_ceil_div(p.nblk, 8) * 8 * p.mblk);
+  const dim3 grid((unsigned)xcd_grid(p.mblk, p.nblk));
   if constexpr (DT == M3X_BF16) {
     // the tiled plan's shapes in bf16 take the strip kernel (EPI_QKR: when its 256-column blocks hold whole heads)
     constexpr int NG = strip_ng<EPI>();
     if (p.tiled && (EPI != EPI_QKR || N % (64 * NG) == 0)) {
       const int nblk = m3x_ceil_div(m3x_ceil_div(N, 16), 4 * NG);
       const int mblk = m3x_ceil_div(M, 16 * STRIP_RT);
-      hipLaunchKernelGGL((linear_strip_kernel<DT, EPI, PRO, STRIP_RT, NG>), dim3(m3x_ceil_div(nblk, 8) * 8 * mblk),
+      hipLaunchKernelGGL((linear_strip_kernel<DT, EPI, PRO, STRIP_RT, NG>), dim3((unsigned)xcd_grid(mblk, nblk)),
                          dim3(256), 0, st, X, ldx, W, W2, Y, ldy, M, N, K, mblk, nblk, ni, ro, qk);
       return true;
     }
