@@ -3,6 +3,7 @@
 // 16-bit with fp32 arithmetic. Every stateful layer keeps one row per slot (the reference's conv_flat / kv /
 // key_pos rows); several padding seats of a batch may name the one dummy slot, whose rows are scratch.
 #include "m3x_common.h"
+#include "m3x_gemm_f32x3.h"
 
 // Stateful kernels split a seat's rows over workgroups (blockIdx.y); the chunk is at least the state's depth, so
 // only chunk 0 reads the old state, and chunk 0 alone writes the new state after a barrier. A thread keeps at
@@ -10,13 +11,6 @@
 constexpr int CODEC_THREADS = 256;
 constexpr int CODEC_KEEP = 16;
 constexpr long NEVER_POS = -(1L << 40);  // key_pos of an empty ring entry
-
-// ELU (alpha 1). 16-bit storage: the hardware exp, exp(v) - 1 for v <= 0, absolute error ~1e-7, below the storage
-// step of every value it produces. fp32 storage: expm1f, accurate to an ulp of the result near 0 as well.
-template <int DT> __device__ __forceinline__ float elu(float v) {
-  if constexpr (DT == M3X_F32) return v > 0.f ? v : expm1f(v);
-  else return v > 0.f ? v : __expf(v) - 1.f;
-}
 
 // ---------------------------------------------------------------------------------------------------------
 // RVQ decode (:134-149; transformers MimiSplitResidualVectorQuantizer.decode): out[b, :dim] = table_0[code_0]
@@ -342,6 +336,148 @@ __global__ __launch_bounds__(256) void conv_gemm_kernel(const Elt<DT>* __restric
         }
         *reinterpret_cast<uint2*>(Y + m * ldy + n) = *reinterpret_cast<const uint2*>(o);
       }
+    }
+  }
+}
+
+// The gathered fp32 conv on the bf16 matrix cores (m3x_gemm_f32x3.h's split and sums; the epilogue as conv_gemm_kernel).
+// conv_gemm_kernel reads a row once per tap and repeats the ELU in front of the conv (about 30 instructions an element)
+// each time, which bounds it. Here a workgroup owns 128 rows of one seat (blockIdx.x = seat x row block, rows past T
+// are dropped) and the 16 CT columns of its column block; per 32 channels it loads the 128 + pad joined rows once,
+// applies the ELU and splits them once into LDS, splits the TAPS x CT weight fragments beside them, and multiplies
+// all taps from LDS: a tap's fragment is the same rows shifted by tap * dil (row r sits in slot r % 16, XOR-swizzled by
+// its k group, of fragment r / 16, so 16 consecutive rows hit 16 bank groups wherever they start). The products add up
+// channel block by channel block, taps within.
+constexpr int CX_ROWS = 128, CX_PAD = 16;  // rows a workgroup, most history frames
+
+template <int CT, int TAPS>
+__global__ __launch_bounds__(256) void conv_x3_kernel(const float* __restrict__ X, long ldx,
+                                                      const float* __restrict__ Wp, float* Y, long ldy, int rblk,
+                                                      F32Epi ep, ConvSrc cs) {
+  constexpr int RT = 2;                               // row tiles a wave: 4 waves x 32 rows
+  constexpr int RF = (CX_ROWS + CX_PAD) / 16;         // row fragments in LDS
+  constexpr int XV = (RF * 64 + 255) / 256;           // 8-float vectors a thread and channel block
+  constexpr int WF = CT * TAPS, WV = (WF + 3) / 4;
+  __shared__ __align__(16) u16x8 lx[3][RF][64], lw[3][WF][64];
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: scalar branches around the MFMAs
+  const int lane = tid & 63;
+  const int li = lane & 15;
+  const int lg = lane >> 4;
+  const int bs = blockIdx.x / rblk;
+  const int t0 = (blockIdx.x - bs * rblk) * CX_ROWS;
+  const int n0 = 16 * CT * blockIdx.y;
+  const int cst = cs.C >> 5;       // channel blocks
+  const int ks = TAPS * cst;
+  const float* xs = X + ((long)bs * cs.T - cs.pad) * ldx;  // joined row i >= pad
+  const float* hs = cs.pad ? (const float*)cs.state + cs.slots[bs] * cs.ld_state : X;
+  const int rows = min(CX_ROWS, cs.T - t0) + cs.pad;       // joined rows t0 .. t0 + rows - 1
+  const int lastw = min(3, (cs.T - t0 - 1) >> 5);          // the waves up to it hold live rows
+  const float* wb = Wp + (long)(n0 >> 4) * ks * 512 + 8 * lane;
+
+  f32x8 xv[XV], wv[WV];
+  auto load = [&](int cb) {
+#pragma unroll
+    for (int j = 0; j < XV; ++j) {
+      const int i = t0 + min((tid >> 2) + 64 * j, rows - 1);  // rows past the block repeat its last (never stored)
+      const int c = 32 * cb + 8 * (tid & 3);
+      xv[j] = ldv<M3X_F32>(i < cs.pad ? hs + (long)i * cs.C + c : xs + (long)i * ldx + c);
+    }
+#pragma unroll
+    for (int j = 0; j < WV; ++j) {
+      const int f = min(wave + 4 * j, WF - 1);  // [tap][tile]
+      wv[j] = ldv<M3X_F32>(wb + ((long)(f % CT) * ks + (f / CT) * cst + cb) * 512);
+    }
+  };
+  f32x4_t acc[CT][RT];
+#pragma unroll
+  for (int a = 0; a < CT; ++a)
+#pragma unroll
+    for (int t = 0; t < RT; ++t) acc[a][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  load(0);
+  for (int cb = 0; cb < cst; ++cb) {
+    __syncthreads();  // every wave is done reading the previous channels
+#pragma unroll
+    for (int j = 0; j < XV; ++j) {
+      const int r = (tid >> 2) + 64 * j;
+      // wave-uniform: the 16 rows that this wave stores, if a live wave reads them
+      if (wave + 4 * j < RF && 16 * (wave + 4 * j) < 32 * (lastw + 1) + cs.pad) {
+        if (cs.pre_elu && t0 + r >= cs.pad) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) xv[j].v[e] = elu<M3X_F32>(xv[j].v[e]);
+        }
+        const int s = 16 * (tid & 3) + ((r & 15) ^ (4 * (tid & 3)));
+        split_bf16x3(xv[j], lx[0][r >> 4][s], lx[1][r >> 4][s], lx[2][r >> 4][s]);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < WV; ++j)
+      if (wave + 4 * j < WF)  // wave-uniform
+        split_bf16x3(wv[j], lw[0][wave + 4 * j][lane], lw[1][wave + 4 * j][lane], lw[2][wave + 4 * j][lane]);
+    __syncthreads();
+    if (cb + 1 < cst) load(cb + 1);
+    if (wave > lastw) continue;
+#pragma unroll
+    for (int tap = 0; tap < TAPS; ++tap) {
+      u16x8 b[RT][3];
+#pragma unroll
+      for (int t = 0; t < RT; ++t) {
+        const int r = 16 * (wave * RT + t) + li + tap * cs.dil;
+        const int s = 16 * lg + ((r & 15) ^ (4 * lg));
+#pragma unroll
+        for (int p = 0; p < 3; ++p) b[t][p] = lx[p][r >> 4][s];
+      }
+#pragma unroll
+      for (int a = 0; a < CT; ++a) {
+        u16x8 w[3];
+#pragma unroll
+        for (int p = 0; p < 3; ++p) w[p] = lw[p][tap * CT + a][lane];
+        mfma_x3<RT>(w, b, acc[a]);
+      }
+    }
+  }
+  if (any_nonfinite<CT, RT>(acc)) {
+#pragma unroll
+    for (int a = 0; a < CT; ++a)
+#pragma unroll
+      for (int t = 0; t < RT; ++t) acc[a][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < ks; ++s) {
+      const int tap = s / cst;
+#pragma unroll
+      for (int t = 0; t < RT; ++t) {
+        const int i = t0 + min(16 * (wave * RT + t) + li + tap * cs.dil, rows - 1);
+        const int c = 32 * (s - tap * cst) + 8 * lg;
+        f32x8 x = ldv<M3X_F32>(i < cs.pad ? hs + (long)i * cs.C + c : xs + (long)i * ldx + c);
+        if (cs.pre_elu && i >= cs.pad) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) x.v[e] = elu<M3X_F32>(x.v[e]);
+        }
+#pragma unroll
+        for (int a = 0; a < CT; ++a)
+          acc[a][t] = mfma16x16x32_f32(ldv<M3X_F32>(wb + ((long)a * ks + s) * 512), x, acc[a][t]);
+      }
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < RT; ++t) {
+    const int tr = t0 + 16 * (wave * RT + t) + li;
+    if (tr >= cs.T) continue;
+    const long m = (long)bs * cs.T + tr;
+#pragma unroll
+    for (int a = 0; a < CT; ++a) {
+      const int n = n0 + 16 * a + 4 * lg;
+      const float4 bb = ep.bias ? *reinterpret_cast<const float4*>(ep.bias + n) : make_float4(0.f, 0.f, 0.f, 0.f);
+      const float4 rr = ep.res ? *reinterpret_cast<const float4*>(ep.res + m * ep.ld_res + n) : make_float4(0.f, 0.f, 0.f, 0.f);
+      const float bv[4] = {bb.x, bb.y, bb.z, bb.w}, rv[4] = {rr.x, rr.y, rr.z, rr.w};
+      float o[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        float v = acc[a][t][r];
+        if (ep.bias) v = v + bv[r];
+        if (ep.res) v = rv[r] + v;
+        o[r] = ep.use_elu ? elu<M3X_F32>(v) : v;
+      }
+      *reinterpret_cast<float4*>(Y + m * ldy + n) = make_float4(o[0], o[1], o[2], o[3]);
     }
   }
 }
@@ -907,6 +1043,35 @@ M3X_API int m3x_conv_gemm(const void* x, long ldx, const void* w_packed, const v
   const dim3 grid(gx, ny);
   if (dtype == M3X_F32 && bias && !m3x_aligned16(bias)) return M3X_EINVAL;
   hipStream_t st = (hipStream_t)stream;
+  if (dtype == M3X_F32) {
+    const F32Epi ep{(const float*)bias, (const float*)res, ld_res, use_elu};
+    const float *X = (const float*)x, *W = (const float*)w_packed;
+    // conv_x3_kernel: whole channel blocks, 3 taps, 32 or 64 columns a workgroup, at least 70 % of its 128-row blocks'
+    // rows live, enough workgroups for the chip; reads of x overlapping its own output (y = x in place) are out
+    const int rblk = G ? m3x_ceil_div(T, CX_ROWS) : 0, ncol = N == 32 ? 32 : 64;
+    if (G && C % 32 == 0 && K == 3 * C && cs.pad <= CX_PAD && N >= 32 && 10L * T >= 7L * rblk * CX_ROWS && y != x &&
+        (long)(M / T) * rblk * (N / ncol) >= F32X3_MIN_BLOCKS) {
+      const dim3 gx3((unsigned)((long)(M / T) * rblk), N / ncol);
+      if (ncol == 32)
+        hipLaunchKernelGGL((conv_x3_kernel<2, 3>), gx3, dim3(256), 0, st, X, ldx, W, (float*)y, ldy, rblk, ep, cs);
+      else
+        hipLaunchKernelGGL((conv_x3_kernel<4, 3>), gx3, dim3(256), 0, st, X, ldx, W, (float*)y, ldy, rblk, ep, cs);
+      M3X_CHECK_LAUNCH();
+      return M3X_OK;
+    }
+    // plain rows (a 1x1 conv, or gathered columns): the projection's kernel with the conv epilogue
+    const int mblk = m3x_ceil_div(M, 64), nblk = N / 64;
+    if (!G && N >= 64 && y != x && (long)mblk * nblk >= F32X3_MIN_BLOCKS) {
+      if (N == 128)
+        hipLaunchKernelGGL((linear_f32x3_kernel<2, 2, 4, 2>), dim3((unsigned)xcd_grid(mblk, 1)), dim3(256), 0, st, X, ldx,
+                           W, (float*)y, ldy, M, N, K, mblk, 1, ep);
+      else
+        hipLaunchKernelGGL((linear_f32x3_kernel<2, 2, 2, 2>), dim3((unsigned)xcd_grid(mblk, nblk)), dim3(256), 0, st, X,
+                           ldx, W, (float*)y, ldy, M, N, K, mblk, nblk, ep);
+      M3X_CHECK_LAUNCH();
+      return M3X_OK;
+    }
+  }
 #define CG_CASE(DTT, NTT, MTT)                                                                                   \
   if (dtype == DTT && nt == NTT && mt == MTT) {                                                              \
     using ET = Elt<DTT>;                                                                                         \

@@ -1,6 +1,7 @@
 // Projections: the pack kernel, the fp32 projection kernel and the C entry points of the plain and gated
 // projections (the 16-bit kernels and their plans are in m3x_gemm.h).
 #include "m3x_gemm.h"
+#include "m3x_gemm_f32x3.h"
 
 template <int DT>
 __global__ __launch_bounds__(256) void pack_weight_kernel(const Elt<DT>* __restrict__ W, long ldw, int N, int K,
@@ -201,12 +202,34 @@ __global__ __launch_bounds__(256) void linear_f32_kernel(const float* __restrict
   }
 }
 
-// fp32 tile choice: the largest tile (most operand reuse) that still gives at least 256 workgroups; small grids
-// split K four ways.
+// fp32 tile choice. From F32X3_MIN_BLOCKS workgroups of 64 x 64 (rows beyond one 32-row block) the plain and GELU
+// projections take linear_f32x3_kernel, which has no K split and needs the chip mostly filled: at 168 workgroups
+// (448 x 1536 x 512) 13.5 against 14.6 us, at 128 (1000 x 512 x 512) 13.0 against 10.1; from F32X3_WIDE_BLOCKS of them in
+// 64 x 128 tiles: 448 blocks (448 x 8192 x 1024) 53 against 58 us with 64 x 64 and 81 with the fp32 instructions, 320
+// blocks (300 x 8192 x 1024) 49 against 43.5. Larger shapes, fp32 instructions against it: 3584 x 3072 x 512 122 / 79 us,
+// 21504 x 1280 x 256 150 / 101, 107520 x 512 x 128 156 / 120 (MI355X, graph-timed). Below it, and for SwiGLU, the fp32
+// instructions: the largest tile (most operand reuse) that still gives at least 256 workgroups; small grids split K
+// four ways.
+constexpr long F32X3_WIDE_BLOCKS = 440;
+
 template <int EPI>
 static bool launch_linear_f32(hipStream_t st, const float* X, long ldx, const float* W, const float* W2, float* Y,
                               long ldy, int M, int N, int K) {
   const int ntiles = m3x_ceil_div(N, 16);
+  if constexpr (EPI != EPI_SWIGLU) {
+    const int mblk = m3x_ceil_div(M, 64), nblk = m3x_ceil_div(N, 64), nwide = m3x_ceil_div(N, 128);
+    const F32Epi ep{};
+    if (M > 32 && (long)mblk * nblk >= F32X3_MIN_BLOCKS) {
+      if (xcd_grid(mblk, nblk) > 0x7fffffffL) return false;
+      if ((long)mblk * nwide >= F32X3_WIDE_BLOCKS)
+        hipLaunchKernelGGL((linear_f32x3_kernel<2, 2, 4, EPI == EPI_GELU>), dim3((unsigned)xcd_grid(mblk, nwide)),
+                           dim3(256), 0, st, X, ldx, W, Y, ldy, M, N, K, mblk, nwide, ep);
+      else
+        hipLaunchKernelGGL((linear_f32x3_kernel<2, 2, 2, EPI == EPI_GELU>), dim3((unsigned)xcd_grid(mblk, nblk)),
+                           dim3(256), 0, st, X, ldx, W, Y, ldy, M, N, K, mblk, nblk, ep);
+      return true;
+    }
+  }
   const int cand[6][2] = {{4, 4}, {2, 4}, {2, 2}, {1, 4}, {1, 2}, {1, 1}};
   int mt = 1, nw = 1;
   for (const auto& c : cand) {
@@ -223,7 +246,9 @@ static bool launch_linear_f32(hipStream_t st, const float* X, long ldx, const fl
   hipLaunchKernelGGL((linear_f32_kernel<MTT, NWW, EPI>), grid, dim3(256), 0, st, X, ldx, W, W2, Y, ldy, M, N, K, \
                      mblk, nblk)
   switch (mt * 10 + nw) {
-    case 44: M3X_LF(4, 4); return true;
+    case 44:
+      if constexpr (EPI == EPI_SWIGLU) M3X_LF(4, 4);  // 256 such tiles of the others take the kernel above
+      return EPI == EPI_SWIGLU;
     case 24: M3X_LF(2, 4); return true;
     case 22: M3X_LF(2, 2); return true;
     case 14: M3X_LF(1, 4); return true;

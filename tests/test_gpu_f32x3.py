@@ -1,0 +1,96 @@
+"""float32 products on the bf16 matrix cores (three bf16 values an operand): projections and the codec's thin convs at the
+edges of their tiles and of the rules that choose them, against 64-bit products.
+
+Bound, per output, with S = sum_k |x_k w_k|: every accumulator addition rounds by at most 2^-24 of a partial sum (<= S),
+6 per 32 products, the products left out are below 2^-25 S, and an input that went through ELU is off by an ulp."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+pytestmark = pytest.mark.gpu
+
+
+def _bound(s, K, extra=4):
+    return (6 * K / 32 + extra) * 2.0 ** -24 * s + 1e-37
+
+
+def _g(seed):
+    return torch.Generator().manual_seed(seed)
+
+
+@pytest.mark.parametrize("M,N,K", [(64, 10240, 64), (65, 5120, 32), (2500, 257, 96), (10304, 64, 64), (3000, 330, 160),
+                                   (33, 10300, 64), (14080, 128, 32), (28200, 100, 32), (127, 5120, 512)])
+@pytest.mark.parametrize("gelu", [False, True])
+def test_linear_f32x3(gpu, M, N, K, gelu):
+    from m3x import ops
+    g = _g(M + N + K)
+    x = torch.randn(M, K, generator=g).to(gpu)
+    w = (torch.randn(N, K, generator=g) * K ** -0.5).to(gpu)
+    pw = ops.pack_weight(w)
+    y = torch.full((M, N + 4), 7.0, device=gpu)[:, :N] if N % 4 == 0 else torch.full((M, N), 7.0, device=gpu)
+    if gelu:
+        ops.linear_act(x, pw, None, ops.ACT_GELU, y)
+    else:
+        ops.linear(x, pw, y)
+    ref = x.double() @ w.double().t()
+    bound = _bound(x.double().abs() @ w.double().abs().t(), K)
+    if gelu:  # |gelu'| < 1.13; erf and its products a few ulp
+        ref = F.gelu(ref)
+        bound = 1.13 * bound + 2.0 ** -21 * ref.abs() + 2.0 ** -22
+    assert bool(((y.double() - ref).abs() <= bound).all())
+
+
+def test_linear_f32x3_nonfinite(gpu):
+    """Rows with infinities, NaN or values that bf16 rounds to infinity get what fp32 products give; the others are as
+    without them."""
+    from m3x import ops
+    M, N, K = 700, 1024, 64
+    g = _g(5)
+    x = torch.randn(M, K, generator=g)
+    x[3, 5], x[70, 0], x[131, 63], x[200, 7] = float("inf"), float("-inf"), float("nan"), 3.4e38
+    w = (torch.randn(N, K, generator=g) * 0.1).abs() + 0.01
+    x, w = x.to(gpu), w.to(gpu)
+    y = ops.linear(x, ops.pack_weight(w))
+    ref = x.double() @ w.double().t()
+    assert bool((y[3] == float("inf")).all()) and bool((y[70] == float("-inf")).all()) and bool(y[131].isnan().all())
+    assert torch.allclose(y[200].double(), ref[200], rtol=1e-6)
+    rows = [r for r in range(M) if r not in (3, 70, 131, 200)]
+    bound = _bound(x[rows].double().abs() @ w.double().abs().t(), K)
+    assert bool(((y[rows].double() - ref[rows]).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("B,T,C,N,dil,pre", [(160, 96, 64, 64, 1, True), (80, 200, 32, 32, 1, True),
+                                             (40, 480, 128, 64, 1, True), (100, 128, 32, 128, 8, False),
+                                             (161, 97, 64, 32, 3, True), (20, 1000, 32, 64, 1, False),
+                                             (90, 130, 32, 64, 1, True),  # half-empty row blocks: the fp32 kernel
+                                             (7, 96, 64, 64, 1, True)])   # few workgroups: the fp32 kernel
+def test_conv_gemm_f32_gathered(gpu, B, T, C, N, dil, pre):
+    from m3x import ops
+    g = _g(B + T + C + N)
+    k, pad = 3, 2 * dil
+    x = torch.randn(B * T, C, generator=g).to(gpu)
+    state = torch.randn(B + 2, pad * C + 8, generator=g).to(gpu)
+    slots = torch.randperm(B + 2, generator=g)[:B].to(gpu)
+    w = (torch.randn(N, k * C, generator=g) * (k * C) ** -0.5).to(gpu)
+    bias, res = torch.randn(N, generator=g).to(gpu), torch.randn(B * T, N, generator=g).to(gpu)
+    y = res.clone()
+    ops.conv_gemm(x, ops.pack_weight(w), y, bias=bias, res=y, use_elu=True, gather=(state[:, :pad * C], slots, T, C, dil, pre))
+    xd = x.double().view(B, T, C)
+    j = torch.cat([state[slots, :pad * C].double().view(B, pad, C), F.elu(xd) if pre else xd], 1)
+    cols = torch.cat([j[:, i * dil:i * dil + T] for i in range(k)], 2).view(B * T, k * C)
+    pre_act = cols @ w.double().t() + bias.double() + res.double()
+    bound = _bound(cols.abs() @ w.double().abs().t() + bias.double().abs() + res.double().abs(), k * C, 10) + 2.0 ** -22
+    assert bool(((y.double() - F.elu(pre_act)).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("M,N,K", [(10240, 64, 32), (10303, 64, 96), (5130, 128, 64), (16000, 128, 32)])
+def test_conv_gemm_f32_plain(gpu, M, N, K):
+    from m3x import ops
+    g = _g(M + N + K)
+    x = torch.randn(M, K, generator=g).to(gpu)
+    w = (torch.randn(N, K, generator=g) * K ** -0.5).to(gpu)
+    bias, y = torch.randn(N, generator=g).to(gpu), torch.randn(M, N, generator=g).to(gpu)
+    ref = x.double() @ w.double().t() + bias.double() + y.double()
+    bound = _bound(x.double().abs() @ w.double().abs().t() + bias.double().abs() + y.double().abs(), K, 10) + 2.0 ** -22
+    ops.conv_gemm(x, ops.pack_weight(w), y, bias=bias, res=y, use_elu=True)
+    assert bool(((y.double() - F.elu(ref)).abs() <= bound).all())
