@@ -154,8 +154,9 @@ int m3x_linear_normed(const void* x, long ldx, const void* part, const float* u,
  * [(heads + 2 kv_heads) * 128, K] packed, or, when part is given (K = 1024), m3x_linear_normed's RMSNorm-folded
  * product of rows whose tile statistics are part (eps_in the input norm's epsilon, W packed from the folded
  * weight). When the row count's plan gives each workgroup whole heads (193..256 rows and above 512 at N = 4096,
- * K = 1024) the norm, RoPE and cache writes run in the projection's epilogue and qkv is not written; otherwise the
- * two launches run in turn through qkv [M, ld_qkv]. The outputs are the same bits either way.
+ * K = 1024) the norm, RoPE and cache writes run in the projection's epilogue and qkv is not written; otherwise qkv
+ * [M, ld_qkv] holds the projection: up to 192 rows the two launches run in turn through it, at 257..512 the one launch
+ * stores it as well. The outputs are the same bits either way.
  * Replaces `F.linear(x, wqkv)` + `_qk_norm_rope_cache` (serve/fast_backbone.py:193-197, 61-92). */
 int m3x_linear_qk_rope(const void* x, long ldx, const void* part, float eps_in, const void* w_packed, void* qkv,
                        long ld_qkv, void* q_out, long s_qo_b, long s_qo_h, void* k_cache, void* v_cache, long sk_s,

@@ -203,13 +203,14 @@ __global__ __launch_bounds__(256) void linear_f32_kernel(const float* __restrict
 }
 
 // fp32 tile choice. From F32X3_MIN_BLOCKS workgroups of 64 x 64 (rows beyond one 32-row block) the plain and GELU
-// projections take linear_f32x3_kernel, which has no K split and needs the chip mostly filled: at 168 workgroups
-// (448 x 1536 x 512) 13.5 against 14.6 us, at 128 (1000 x 512 x 512) 13.0 against 10.1; from F32X3_WIDE_BLOCKS of them in
-// 64 x 128 tiles: 448 blocks (448 x 8192 x 1024) 53 against 58 us with 64 x 64 and 81 with the fp32 instructions, 320
-// blocks (300 x 8192 x 1024) 49 against 43.5. Larger shapes, fp32 instructions against it: 3584 x 3072 x 512 122 / 79 us,
-// 21504 x 1280 x 256 150 / 101, 107520 x 512 x 128 156 / 120 (MI355X, graph-timed). Below it, and for SwiGLU, the fp32
-// instructions: the largest tile (most operand reuse) that still gives at least 256 workgroups; small grids split K
-// four ways.
+// projections take linear_f32x3_kernel, which has no K split and needs the chip filled: with weights that the launch
+// before did not leave in the caches, 448 x 2048 x 512 (224 workgroups) took 19.4 us against 16.1 and 448 x 1536 x 512
+// (168) 17.6 against 14.2 inside the Mimi frame, though 13.4 against 14.9 and 14.7 when repeated alone. From
+// F32X3_WIDE_BLOCKS of them in 64 x 128 tiles: 448 blocks (448 x 8192 x 1024) 53 against 58 us with 64 x 64 and 81 with the fp32
+// instructions, 320 blocks (300 x 8192 x 1024) 49 against 43.5. Larger shapes, fp32 instructions against it: 3584 x
+// 3072 x 512 122 / 79 us, 21504 x 1280 x 256 150 / 101, 107520 x 512 x 128 156 / 120 (MI355X, graph-timed). Below it, and for
+// SwiGLU, the fp32 instructions: the largest tile (most operand reuse) that still gives at least 256 workgroups; small
+// grids split K four ways.
 constexpr long F32X3_WIDE_BLOCKS = 440;
 
 template <int EPI>

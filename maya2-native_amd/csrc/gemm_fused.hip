@@ -89,8 +89,9 @@ M3X_API int m3x_qk_norm_rope_cache(const void* qkv, long s_qkv, void* q_out, lon
 
 // The q|k|v projection (plain, or with the input norm folded in when part is given: m3x_linear_normed with
 // RMSNorm) followed by m3x_qk_norm_rope_cache on its output, in one launch when the row count's plan holds whole
-// heads per workgroup (193..256 rows and above 512 at N = 4096); otherwise the two launches in turn, through qkv.
-// Same bits either way.
+// heads per workgroup (above 192 rows at N = 4096); otherwise the two launches in turn, through qkv. Same bits either
+// way. qkv holds the projection at up to 192 and at 257..512 rows (there the one launch stores it beside its outputs),
+// and is left alone at the others.
 M3X_API int m3x_linear_qk_rope(const void* x, long ldx, const void* part, float eps_in, const void* w_packed, void* qkv,
                                long ld_qkv, void* q_out, long s_qo_b, long s_qo_h, void* k_cache, void* v_cache,
                                long sk_s, long sk_h, long sk_t, const int64_t* slots, const int32_t* pos,
@@ -118,9 +119,10 @@ M3X_API int m3x_linear_qk_rope(const void* x, long ldx, const void* part, float 
   const uint16_t* X = (const uint16_t*)x;
   const uint16_t* W = (const uint16_t*)w_packed;
   uint16_t* Y = (uint16_t*)qkv;
-  const bool fused = part ? launch_linear<M3X_BF16, EPI_QKR, true>(p, st, X, ldx, W, nullptr, Y, ld_qkv, M, N, K, ni,
+  uint16_t* const Yf = M > 256 && M <= 512 ? Y : nullptr;
+  const bool fused = part ? launch_linear<M3X_BF16, EPI_QKR, true>(p, st, X, ldx, W, nullptr, Yf, ld_qkv, M, N, K, ni,
                                                                    ResidOut{}, qk)
-                          : launch_linear<M3X_BF16, EPI_QKR, false>(p, st, X, ldx, W, nullptr, Y, ld_qkv, M, N, K,
+                          : launch_linear<M3X_BF16, EPI_QKR, false>(p, st, X, ldx, W, nullptr, Yf, ld_qkv, M, N, K,
                                                                     ni, ResidOut{}, qk);
   if (fused) {
     M3X_CHECK_LAUNCH();

@@ -32,8 +32,8 @@
 //   EPI_QKR     the q|k|v projection's values (rounded to bf16 as EPI_NONE stores them) go through the per-head
 //               q/k RMSNorm + RoPE and into the caches (m3x_qk_norm_rope_cache's arithmetic, qk_norm_rope8):
 //               query heads to q_out, key and value heads into the static cache at [slot, head, pos]. Needs whole
-//               heads per workgroup: the large-M tiled plan (128 x 128 tiles) and the one-shot plan with NW = 8 and
-//               one K slice (128 columns).
+//               heads per workgroup: the strip kernel (128- or 256-column blocks) and the one-shot plan with NW = 8
+//               and one K slice (128 columns).
 //
 // Folded norm (PRO): the consumer of a residual row multiplies the raw row and applies the norm to the product.
 // A norm's elementwise weight w (and LayerNorm bias b) is folded into the consumer's weight when it is packed:
@@ -850,232 +850,15 @@ __global__ __launch_bounds__(64 * NWAVES) void linear_oneshot_kernel(const uint1
   }
 }
 
-// Large-M projections (M > 512 rows: steps with inline prefills). A workgroup of 8 waves owns a 2-D tile of 128 (or
-// 96: RT = 3) activation rows x 128 weight rows (for SwiGLU: 64 gate rows from W and the same 64 up rows from W2, i.e. 64
-// output columns) and walks K in stages of 64. The packed weight fragments of a stage are copied to LDS as they are
-// (16 fragments of 1 KB: every fragment read is one contiguous 1 KB); the activation rows sit row-major with a
-// 144-byte row stride, so the 16 rows of a fragment read fall in 16 different bank groups and a row's 8 stores in
-// distinct banks. The waves are 2 x 4 blocks of 16 RT activation rows x 32 weight rows (RT x 2 MFMA tiles; with
-// SwiGLU a wave holds one gate tile and the matching up tile). Stages are double-buffered in LDS: the next stage's
-// global loads are in flight while the current one multiplies, with one barrier per stage. Every weight byte is
-// read by ceil(M / 32 RT) workgroups and every activation byte by ceil(N / 128), against 36 and 64 for the 64 x 64
-// chunked tiles at 2264 rows. Global loads run two stages ahead of the products (three register sets in turn):
-// measured 2-10 % faster than one stage ahead, most on the N = 1024 shapes whose grid has one workgroup per CU.
-// PRO (K == PRO_K): the rows' folded norm, applied in the epilogue; its statistics (and EPI_RESID's operands) load
-// after the products.
-template <int DT, int EPI, bool PRO, int RT>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) void linear_tiled_kernel(const uint16_t* __restrict__ X, long ldx,
-                                                              const uint16_t* __restrict__ Wp,
-                                                              const uint16_t* __restrict__ W2p,
-                                                              uint16_t* __restrict__ Y, long ldy, int M, int N, int K,
-                                                              int mblk, int nblk, NormIn ni, ResidOut ro, QkOut qk) {
-  constexpr bool DUAL = EPI == EPI_SWIGLU;
-  constexpr int BM = 32 * RT;  // activation rows: 2 wave rows x RT tiles of 16
-  static_assert(RT == 3 || RT == 4, "96- or 128-row blocks");
-  constexpr int LDA = 72;  // activation row stride in LDS, halfwords
-  __shared__ __align__(16) uint16_t lw[2][16 * 512];
-  __shared__ __align__(16) uint16_t la[2][BM * LDA];
-  __shared__ float2 pst[PRO ? BM : 1];
-
-  int mb, nb;
-  if (!xcd_block(mblk, nblk, mb, nb)) return;  // padding block: the whole workgroup leaves before any barrier
-
-  const int tid = threadIdx.x;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int lane = tid & 63;
-  const int li = lane & 15;
-  const int lg = lane >> 4;
-  const int wm = wave & 1;   // activation tiles RT wm .. RT wm + RT - 1
-  const int wn = wave >> 1;  // weight tiles (below)
-  const int ksteps = K >> 5;
-  const int ntiles = (N + 15) >> 4;
-  const int m0 = mb * BM;
-  NormStage<BM, 512, PRO_K / 128> ns;
-
-  // per-thread load slots: vector v = tid + 512 j of a stage; weights: fragment f = v / 64 = tid / 64 + 8 j (tile
-  // t = f / 2, step f % 2), lane v % 64, at LDS 8 v; activations: row v / 8 = tid / 8 + 64 j, 16-byte column v % 8.
-  // Offsets are 32-bit element offsets; with SwiGLU, slot j = 0 holds gate rows and j = 1 up rows.
-  int gw[2], ga[2];
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int f = (tid >> 6) + 8 * j;
-    const int t = f >> 1, st = f & 1;
-    const int tt = min(DUAL ? nb * 4 + (t & 3) : nb * 8 + t, ntiles - 1);  // tiles past N: valid, never stored
-    gw[j] = (tt * ksteps + st) * 512 + (tid & 63) * 8;
-    // rows past M: re-read, never stored; with 96-row blocks the second slot's rows past the block repeat its
-    // last row (the same value to the same LDS place)
-    ga[j] = min(m0 + min((tid >> 3) + 64 * j, BM - 1), M - 1) * (int)ldx + 8 * (tid & 7);
-  }
-  int la0[2];
-#pragma unroll
-  for (int j = 0; j < 2; ++j) la0[j] = min((tid >> 3) + 64 * j, BM - 1) * LDA + 8 * (tid & 7);
-  // the wave's 2 weight tiles: plain 2 wn + i; SwiGLU gate wn and up 4 + wn
-  int wt[2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i) wt[i] = DUAL ? (i == 0 ? wn : 4 + wn) : 2 * wn + i;
-
-  f32x4_t acc[2][RT];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < RT; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-
-  // a stage's loads in r[0..1] (weight fragments) and r[2..3] (activation rows); stages past the end re-read the
-  // last stage (valid addresses, never stored)
-  const int nst = K >> 6;
-  auto gload = [&](int stg, u16x8(&r)[4]) {
-    const int sc = min(stg, nst - 1);
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      r[j] = ld16((DUAL && j == 1 ? W2p : Wp) + gw[j] + sc * 1024);
-      r[2 + j] = ld16(X + ga[j] + sc * 64);
-    }
-  };
-  auto lstore = [&](int buf, const u16x8(&r)[4]) {
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      st16(&lw[buf][tid * 8 + 4096 * j], r[j]);
-      st16(&la[buf][la0[j]], r[2 + j]);
-    }
-  };
-  auto compute = [&](int buf) {
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      u16x8 a[2], b[RT];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) a[i] = *reinterpret_cast<const u16x8*>(&lw[buf][(wt[i] * 2 + s) * 512 + lane * 8]);
-#pragma unroll
-      for (int j = 0; j < RT; ++j)
-        b[j] = *reinterpret_cast<const u16x8*>(&la[buf][(16 * (RT * wm + j) + li) * LDA + 32 * s + 8 * lg]);
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < RT; ++j) acc[i][j] = mfma16x16x32<DT>(a[i], b[j], acc[i][j]);
-    }
-  };
-  u16x8 R0[4], R1[4], R2[4];
-  gload(0, R0);
-  gload(1, R1);
-  lstore(0, R0);
-  __syncthreads();
-  // Stage s issues the loads of stage s + 2, multiplies stage s from LDS buffer s % 2 and stores stage s + 1
-  // (loaded during stage s - 1) to the other buffer: every load has two stages of products to arrive in. Three
-  // register sets rotate with the stage, so the loop is unrolled by 6 (register set s % 3, buffer s % 2).
-#define M3X_TILED_STAGE(S, RN, RS, BUF)        \
-  if (s0 + S < nst) {                          \
-    gload(s0 + S + 2, RN);                     \
-    compute(BUF);                              \
-    if (s0 + S + 1 < nst) lstore(BUF ^ 1, RS); \
-    __syncthreads();                           \
-  }
-  for (int s0 = 0; s0 < nst; s0 += 6) {
-    M3X_TILED_STAGE(0, R2, R1, 0)
-    M3X_TILED_STAGE(1, R0, R2, 1)
-    M3X_TILED_STAGE(2, R1, R0, 0)
-    M3X_TILED_STAGE(3, R2, R1, 1)
-    M3X_TILED_STAGE(4, R0, R2, 0)
-    M3X_TILED_STAGE(5, R1, R0, 1)
-  }
-#undef M3X_TILED_STAGE
-
-  // the epilogue's operands load after the products: held across the long K loop they would cost the registers
-  // of a second workgroup per CU
-  ResidPre pre[2][RT];
-  if constexpr (EPI == EPI_RESID) {
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < RT; ++j)
-        pre[i][j] = resid_prefetch(ro, m0 + 16 * (RT * wm + j) + li, (nb * 8 + wt[i]) * 16 + 4 * lg, M, N);
-  }
-  if constexpr (PRO) ns.load(ni, m0, M, PRO_K);
-
-  if constexpr (PRO) {
-    ns.finish(ni, m0, M, PRO_K, pst);  // the rows' scale and shift, from statistics that arrived long ago
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int n = DUAL ? (nb * 4 + wn) * 16 + 4 * lg : (nb * 8 + wt[i]) * 16 + 4 * lg;
-#pragma unroll
-      for (int j = 0; j < RT; ++j) norm_apply(acc[i][j], pst, 16 * (RT * wm + j) + li, ni, n, N, DUAL ? i : 0);
-    }
-  }
-  if constexpr (EPI == EPI_RESID) {
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int tile = nb * 8 + wt[i];
-#pragma unroll
-      for (int j = 0; j < RT; ++j)
-        resid_quad<DT>(acc[i][j], pre[i][j], m0 + 16 * (RT * wm + j) + li, tile * 16 + 4 * lg, tile, M, N, lg, ro, Y,
-                       ldy);
-    }
-    return;
-  }
-  if constexpr (EPI == EPI_QKR) {
-    // the workgroup's 128 columns are one head: stage the 128 x 128 tile in the activation buffers (free after the
-    // loop's last barrier), then the per-head norm, RoPE and cache writes
-    static_assert(DT == M3X_BF16 && BM * (128 + 8) <= 2 * BM * LDA, "the staged tile fits the activation buffers");
-    constexpr int LDT = 128 + 8;
-    uint16_t* tile = &la[0][0];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < RT; ++j) qk_stage(tile, LDT, 16 * (RT * wm + j) + li, 16 * wt[i] + 4 * lg, acc[i][j]);
-    __syncthreads();
-    qk_items<BM, 1, 512>(tile, LDT, nb, m0, M, qk);
-    return;
-  }
-
-  // epilogue: lane (li, lg) of tile pair (i, j) holds weight rows 4 lg + r of tile wt[i] for activation row
-  // m0 + 16 (RT wm + j) + li
-  const bool vec = (ldy & 3) == 0 && (((uintptr_t)Y) & 7) == 0;
-  constexpr int NI = DUAL ? 1 : 2;
-#pragma unroll
-  for (int i = 0; i < NI; ++i) {
-    const int n = DUAL ? (nb * 4 + wn) * 16 + 4 * lg : (nb * 8 + wt[i]) * 16 + 4 * lg;
-#pragma unroll
-    for (int j = 0; j < RT; ++j) {
-      const int m = m0 + 16 * (RT * wm + j) + li;
-      if (m >= M) continue;
-      uint16_t o[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        float v = rnd<DT>(acc[i][j][r]);
-        if constexpr (DUAL) {
-          const float g = v;
-          const float u = rnd<DT>(acc[1][j][r]);
-          v = rnd<DT>(silu16(g)) * u;
-        } else if constexpr (EPI == EPI_GELU) {
-          v = 0.5f * v * (1.0f + erff(v * 0.70710678118654752f));
-        }
-        o[r] = E<DT>::from_f(v);
-      }
-      uint16_t* yp = Y + (long)m * ldy + n;
-      if (vec && n + 3 < N) {
-        uint2 pk;
-        pk.x = (uint32_t)o[0] | ((uint32_t)o[1] << 16);
-        pk.y = (uint32_t)o[2] | ((uint32_t)o[3] << 16);
-        *reinterpret_cast<uint2*>(yp) = pk;
-      } else {
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (n + r < N) yp[r] = o[r];
-      }
-    }
-  }
-}
-
-// Large-M projections in bf16, column strips (M > 512 rows; preferred over linear_tiled_kernel where an instance
-// exists). A workgroup of 4 waves owns BM = 16 RT activation rows x 4 strips of NG weight tiles: wave w's strip is
-// tiles (4 nb + w) NG .. + NG - 1 (16 NG columns; with SwiGLU NG gate tiles and the same NG up tiles). A wave loads
-// its strip's packed fragments from global memory straight into its registers (a fragment is one contiguous 1 KB
-// that no other wave of the workgroup reads), two K stages of 64 ahead in three register sets; only the activation
-// rows pass through LDS (double-buffered, 144-byte row stride), where all 4 waves read them. Against the 2-D tiles
-// of linear_tiled_kernel, where every wave reads both operands from LDS, this cuts the LDS traffic per product by
-// more than half (measured at 2264 rows: waves waiting on LDS issue 27 % -> 3 % of their cycles; q|k|v 34 -> 27.5
-// us, gate|up + SwiGLU 47 -> 40 us, down 38 -> 28 us with its substep-pipelined reads). Products accumulate in the same K order with the same MFMA as
-// linear_tiled_kernel, so the two kernels give the same bits. Epilogues as linear_tiled_kernel's; EPI_QKR needs
-// BN = 64 NG to hold whole heads of 128 columns (2 per workgroup at NG = 4).
+// Projections of many rows, column strips (strip_tile chooses the tile, and when). A workgroup of 4 waves owns BM = 16 RT
+// activation rows x 4 strips of NG weight tiles: wave w's strip is tiles (4 nb + w) NG .. + NG - 1 (16 NG columns; with
+// SwiGLU NG gate tiles and the same NG up tiles). A wave loads its strip's packed fragments from global memory straight
+// into its registers (a fragment is one contiguous 1 KB that no other wave of the workgroup reads), two K stages of 64
+// ahead in three register sets; only the activation rows pass through LDS (double-buffered, 144-byte row stride, so the
+// 16 rows of a fragment read fall in 16 bank groups), where all 4 waves read them. Small tiles are bound by the chain of
+// a stage (LDS store, barrier, LDS read, products: ~500 cycles; three to five stages ahead instead of two were no
+// faster), large ones by the CU's L1 path. K order is the same for every tile: the tile does not change the bits.
+// EPI_QKR needs BN = 64 NG to hold whole heads of 128 columns.
 template <int DT, int EPI, bool PRO, int RT, int NG>
 __global__ __launch_bounds__(256) void linear_strip_kernel(const uint16_t* __restrict__ X, long ldx,
                                                           const uint16_t* __restrict__ Wp,
@@ -1242,7 +1025,7 @@ __global__ __launch_bounds__(256) void linear_strip_kernel(const uint16_t* __res
   }
 #undef M3X_STRIP_STAGE
 
-  // the epilogue's operands load after the products, as in linear_tiled_kernel
+  // the epilogue's operands load after the products: before them they would cost registers through the K loop
   ResidPre pre[EPI == EPI_RESID ? NG : 1][RT];
   if constexpr (EPI == EPI_RESID) {
 #pragma unroll
@@ -1275,7 +1058,12 @@ __global__ __launch_bounds__(256) void linear_strip_kernel(const uint16_t* __res
 #pragma unroll
     for (int i = 0; i < NG; ++i)
 #pragma unroll
-      for (int j = 0; j < RT; ++j) qk_stage(tile, LDT, 16 * j + li, 16 * (wave * NG + i) + 4 * lg, acc[0][i][j]);
+      for (int j = 0; j < RT; ++j) {
+        qk_stage(tile, LDT, 16 * j + li, 16 * (wave * NG + i) + 4 * lg, acc[0][i][j]);
+        const int m = m0 + 16 * j + li;
+        if (Y && m < M)  // the projection itself, for callers that read it (uniform)
+          qk_stage(Y + (long)m * ldy, 0, 0, (t0 + i) * 16 + 4 * lg, acc[0][i][j]);
+      }
     __syncthreads();
     qk_items_staged<BM, BN / 128, 256>(tile, LDT, nb, m0, M, qk, sps, ssl);
     return;
@@ -1316,22 +1104,51 @@ __global__ __launch_bounds__(256) void linear_strip_kernel(const uint16_t* __res
   }
 }
 
-// The strip plan's geometry: 80-row blocks (RT = 5; measured best of 5, 8, 9 and 15 at 2264 and 4096 rows, with two
-// workgroups per CU), 4 weight tiles per wave (2 gate + 2 up pairs with SwiGLU, 2 for the residual projections,
-// whose N = 1024 otherwise leaves too few workgroups).
-constexpr int STRIP_RT = 5;
+// The strip kernel's tile (RT row tiles x 4 NG weight tiles) for M rows of N columns, rt = 0: another plan. The largest
+// of the tiles whose grid keeps the chip busy; graph-timed on MI355X, us (tile: time, blocks in brackets):
+//   plain    2264 x 4096 x 1024: 80 x 256 26.6 (464), 64 x 128 30.5 (1152); 1024 x 4096 x 1024: 16.8 (208), 14.2 (512);
+//            30720 x 512 x 128: 17.8 (768), 19.5 (1920); 3584 x 3072 x 512: 27.2 (540: a second round of two a CU, nearly
+//            empty), 24.6 (1344). So 80 x 256 for one full round or many.
+//            416 x 3072 x 1024 GELU: 32 x 64 10.1 (624), 64 x 64 11.5 (336); 700 x 3072 x 512: 9.4 (1056), 8.7 (528)
+//            1024 x 256 x 1536: 32 x 64 6.5 (128), 64 x 64 8.5 (64), 64 x 128 11.9 (32); 3584 x 256 x 1536: 10.4 (448),
+//            10.3 (224), 12.2 (112)
+//   SwiGLU   1500 x 3072 x 1024: 80-row pairs of strips 24.0 (456), 64 rows x 64 columns 26.8 (1152); 512 rows: 15.8, 12.4
+//   residual 2264 x 1024 x 2048: 80 x 128 21.7 (232), 64 x 64 26.0 (576); 1024 rows: 20.8, 13.2 (256), 32 x 64 13.7 (512);
+//            640 rows: 20.4, 12.0 (160), 11.0 (320)
+// (bf16 at K = 1024 and more, fp16 below.) The 8-wave 128 x 128 tiles with both operands in LDS that such shapes took
+// before were slower at every one of them but 6144 x 1280 x 256 (13.6 against 14.2). Up to 512 rows the K-split plans
+// win unless 32 x 64 blocks fill the chip: 448 x 1536 x 512 4.7 (336 blocks) against 5.2, 448 x 512 x 512 4.0 (112)
+// against 3.3, residual 512 x 1024 x 2048 10.0 (256) against 9.9.
+struct StripTile {
+  int rt, ng;
+};
 template <int EPI>
-constexpr int strip_ng() {
-  return EPI == EPI_SWIGLU || EPI == EPI_RESID ? 2 : 4;
+static StripTile strip_tile(int M, int N, int K, long ldx) {
+  // 32-bit element offsets into the packed weight and the activations; whole K stages
+  if (M <= 256 || K % 64 || (long)m3x_ceil_div(N, 16) * 16 * K >= (1L << 31) || (long)M * ldx >= (1L << 31)) return {0, 0};
+  auto blocks = [&](int rt, int ng) { return (long)m3x_ceil_div(M, 16 * rt) * m3x_ceil_div(N, 64 * ng); };
+  if (M <= 512 && blocks(2, 1) < 300) return {0, 0};
+  if constexpr (EPI == EPI_QKR) {
+    const long b = blocks(5, 4);
+    if (N % 256 == 0 && ((b >= 440 && b <= 512) || b >= 740)) return {5, 4};
+    return N % 128 == 0 ? StripTile{4, 2} : StripTile{0, 0};
+  } else if constexpr (EPI == EPI_SWIGLU) {
+    if (blocks(5, 2) >= 440) return {5, 2};
+  } else if constexpr (EPI == EPI_RESID) {
+    if (blocks(4, 1) > 480) return {5, 2};
+  } else {
+    const long b = blocks(5, 4);
+    if ((b >= 440 && b <= 512) || b >= 740) return {5, 4};
+    if (blocks(4, 2) >= 250) return {4, 2};
+    return blocks(4, 1) >= 400 ? StripTile{4, 1} : StripTile{2, 1};
+  }
+  return blocks(4, 1) >= 200 ? StripTile{4, 1} : StripTile{2, 1};
 }
 
-// Launch geometry: MT activation tiles of 16 rows per workgroup; NW weight tiles per workgroup; NWAVES waves
-// (NWAVES / NW K slices).
 struct LinearPlan {
   int mt, nw, mblk, nblk;
   int nwaves;   // 4 for the chunked kernel and the small one-shot; 8 or 16 for the wide one-shot
   int oneshot;  // steps per K slice for the one-shot kernel, 0 for the chunked kernel
-  int tiled;    // 1: linear_tiled_kernel (M > 512, K % 64 == 0)
 };
 
 // Small one-shot (4 waves): each of the 4/nw K slices is exactly 8 or 16 steps of 32 and the activation block
@@ -1357,8 +1174,16 @@ static bool wide_plan(int M, int N, int K, bool dual, LinearPlan& p) {
     p.oneshot = K / 256;
     return true;
   }
-  if (M < 64 || M > 256) return false;
   const int ntiles = m3x_ceil_div(N, 16);
+  if (M > 256 && M <= 512 && K == 2048 && !dual && (long)m3x_ceil_div(M, 32) * m3x_ceil_div(ntiles, 4) <= 256) {
+    // 32-row blocks of 16 waves in one round (512 x 1024 x 2048 with the residual: 8.5 against 9.9 us chunked)
+    p.mt = 2;
+    p.nw = 4;
+    p.nwaves = 16;
+    p.oneshot = 16;
+    return true;
+  }
+  if (M < 64 || M > 256) return false;
   if (K == 1024) {
     const int cand[4][2] = {{2, 2}, {2, 4}, {3, 4}, {2, 8}};
     for (const auto& c : cand) {
@@ -1393,20 +1218,6 @@ static LinearPlan linear_plan(int M, int N, int K, bool dual, long ldx) {
   auto blocks = [&](int mt, int nw) { return (long)m3x_ceil_div(M, 16 * mt) * m3x_ceil_div(ntiles, nw); };
   LinearPlan p;
   p.nwaves = 4;
-  p.tiled = 0;
-  // tiled: 32-bit element offsets into the packed weight and the activations
-  if (M > 512 && K % 64 == 0 && (long)ntiles * 16 * K < (1L << 31) && (long)M * ldx < (1L << 31)) {
-    p.tiled = 1;
-    p.nw = dual ? 4 : 8;
-    p.oneshot = 0;
-    p.nblk = m3x_ceil_div(ntiles, p.nw);
-    // 96- or 128-row blocks, whichever gives the fewer rows per CU over the rounds of two workgroups per CU
-    // (measured at 2264 rows: 96 is 9-11 % faster for q|k|v, o and down, 11 % slower for gate|up's 1,152 blocks)
-    const long w6 = (long)m3x_ceil_div(M, 96) * p.nblk, w8 = (long)m3x_ceil_div(M, 128) * p.nblk;
-    p.mt = (w6 + 511) / 512 * 96 < (w8 + 511) / 512 * 128 ? 6 : 8;
-    p.mblk = m3x_ceil_div(M, 16 * p.mt);
-    return p;
-  }
   if (wide_plan(M, N, K, dual, p)) {
     p.mblk = m3x_ceil_div(M, 16 * p.mt);
     p.nblk = m3x_ceil_div(ntiles, p.nw);
@@ -1445,43 +1256,32 @@ static bool launch_linear(const LinearPlan& p, hipStream_t st, const uint16_t* X
                           const uint16_t* W2, uint16_t* Y, long ldy, int M, int N, int K, const NormIn& ni = NormIn{},
                           const ResidOut& ro = ResidOut{}, const QkOut& qk = QkOut{}) {
   static_assert(!(PRO && EPI == EPI_RESID), "a residual projection takes its input as is");
-  const dim3 grid((unsigned)xcd_grid(p.mblk, p.nblk));
-  if constexpr (DT == M3X_BF16) {
-    // the tiled plan's shapes in bf16 take the strip kernel (EPI_QKR: when its 256-column blocks hold whole heads)
-    constexpr int NG = strip_ng<EPI>();
-    if (p.tiled && (EPI != EPI_QKR || N % (64 * NG) == 0)) {
-      const int nblk = m3x_ceil_div(m3x_ceil_div(N, 16), 4 * NG);
-      const int mblk = m3x_ceil_div(M, 16 * STRIP_RT);
-      hipLaunchKernelGGL((linear_strip_kernel<DT, EPI, PRO, STRIP_RT, NG>), dim3((unsigned)xcd_grid(mblk, nblk)),
-                         dim3(256), 0, st, X, ldx, W, W2, Y, ldy, M, N, K, mblk, nblk, ni, ro, qk);
-      return true;
+  const StripTile t = strip_tile<EPI>(M, N, K, ldx);
+  if (t.rt) {
+    const int nblk = m3x_ceil_div(N, 64 * t.ng), mblk = m3x_ceil_div(M, 16 * t.rt);
+#define M3X_STRIP(RTT, NGG)                                                                                           \
+  hipLaunchKernelGGL((linear_strip_kernel<DT, EPI, PRO, RTT, NGG>), dim3((unsigned)xcd_grid(mblk, nblk)), dim3(256), 0, \
+                     st, X, ldx, W, W2, Y, ldy, M, N, K, mblk, nblk, ni, ro, qk)
+    constexpr bool WIDE = EPI != EPI_SWIGLU && EPI != EPI_RESID;  // 256-column blocks, else 128
+    if (t.rt == 5) M3X_STRIP(5, (WIDE ? 4 : 2));
+    if constexpr (WIDE) {
+      if (t.ng == 2) M3X_STRIP(4, 2);
     }
+    if constexpr (EPI != EPI_QKR) {
+      if (t.rt == 4 && t.ng == 1) M3X_STRIP(4, 1);
+      if (t.rt == 2) M3X_STRIP(2, 1);
+    }
+#undef M3X_STRIP
+    return true;
   }
+  const dim3 grid((unsigned)xcd_grid(p.mblk, p.nblk));
   if constexpr (EPI == EPI_QKR) {
-    // whole heads per workgroup: the tiled plan (128 columns) or the one-shot plan of 8 weight tiles in one K slice
-    if (p.tiled) {
-      if (p.mt == 6)
-        hipLaunchKernelGGL((linear_tiled_kernel<DT, EPI_QKR, PRO, 3>), grid, dim3(512), 0, st, X, ldx, W, W2, Y, ldy,
-                           M, N, K, p.mblk, p.nblk, ni, ro, qk);
-      else
-        hipLaunchKernelGGL((linear_tiled_kernel<DT, EPI_QKR, PRO, 4>), grid, dim3(512), 0, st, X, ldx, W, W2, Y, ldy,
-                           M, N, K, p.mblk, p.nblk, ni, ro, qk);
-      return true;
-    }
+    // whole heads per workgroup: the one-shot plan of 8 weight tiles in one K slice
     if (!p.oneshot || p.mt != 2 || p.nw != 8 || p.nwaves != 8 || p.oneshot != 32) return false;
     hipLaunchKernelGGL((linear_oneshot_kernel<DT, 2, 8, 8, EPI_QKR, 32, PRO>), grid, dim3(512), 0, st, X, ldx, W, W2,
                        Y, ldy, M, N, K, p.mblk, p.nblk, ni, ro, qk);
     return true;
   } else {
-  if (p.tiled) {
-    if (p.mt == 6)
-      hipLaunchKernelGGL((linear_tiled_kernel<DT, EPI, PRO, 3>), grid, dim3(512), 0, st, X, ldx, W, W2, Y, ldy, M, N,
-                         K, p.mblk, p.nblk, ni, ro, qk);
-    else
-      hipLaunchKernelGGL((linear_tiled_kernel<DT, EPI, PRO, 4>), grid, dim3(512), 0, st, X, ldx, W, W2, Y, ldy, M, N,
-                         K, p.mblk, p.nblk, ni, ro, qk);
-    return true;
-  }
 #define M3X_ONE(MTT, NWW, NWV, SS)                                                                              \
   if constexpr (!PRO || (NWV / NWW) * SS * 32 == PRO_K) {                                                     \
     hipLaunchKernelGGL((linear_oneshot_kernel<DT, MTT, NWW, NWV, EPI, SS, PRO>), grid, dim3(64 * NWV), 0, st, X, \
@@ -1515,6 +1315,7 @@ static bool launch_linear(const LinearPlan& p, hipStream_t st, const uint16_t* X
       case 280832: if constexpr (EPI != EPI_SWIGLU) { M3X_ONE(2, 8, 8, 32); } return false;
       // wide, K = 2048 / 2816 / 3072
       case 141616: if constexpr (EPI != EPI_SWIGLU) { M3X_ONE(1, 4, 16, 16); } return false;
+      case 241616: if constexpr (EPI != EPI_SWIGLU) { M3X_ONE(2, 4, 16, 16); } return false;
       case 121608: if constexpr (EPI != EPI_SWIGLU) { M3X_ONE(1, 2, 16, 8); } return false;
       case 141622: if constexpr (EPI != EPI_SWIGLU) { M3X_ONE(1, 4, 16, 22); } return false;
       case 121611: if constexpr (EPI != EPI_SWIGLU) { M3X_ONE(1, 2, 16, 11); } return false;

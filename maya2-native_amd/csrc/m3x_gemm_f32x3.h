@@ -12,7 +12,7 @@ template <int DT> __device__ __forceinline__ float elu(float v) {
 
 // Workgroups from which the kernels below have the chip filled enough to beat the fp32 instructions with their K splits
 // and smaller tiles (measurements at launch_linear_f32).
-constexpr long F32X3_MIN_BLOCKS = 160;
+constexpr long F32X3_MIN_BLOCKS = 256;
 
 // The conv epilogue: y = act(res + (acc + bias)), bias and res optional, act = ELU when use_elu.
 struct F32Epi {
