@@ -555,17 +555,40 @@ __global__ __launch_bounds__(CODEC_THREADS) void convt_overlap_kernel(const Elt<
 // p - window < key_pos <= p, softmax at scale 1/sqrt(64). qkv rows [q heads | k heads | v heads] (as many kv heads
 // as heads), head_dim 64.
 // TM bounds T at compile time, which keeps the unrolled code small.
-// One 4-wave workgroup per (seat, head). Thread j owns ring entry j for the scores (its key row read whole, the
-// queries read from LDS as broadcasts); the softmax is block-wide; for P.V wave w sums entries 64 w .. 64 w + 63
-// with lane (g, d8) taking keys g (mod 8) and dims 8 d8 .. + 7, all loads in flight at once and no branch around
-// them (masked entries have probability 0); the 8 key groups meet by shuffles and the 4 waves in LDS. Each key
-// and value row is read once for all T queries. The head-0 workgroup records key_pos; every workgroup knows the
-// positions of the entries this call writes, so none depends on another's key_pos write.
+// One 4-wave workgroup per (seat, head), heads fastest: the 8 heads of a seat, whose rows interleave in the ring, run
+// at the same time on the 8 XCDs. Lane (g, d8) of wave w owns dims 8 d8 .. + 7 of ring entries 64 w + g + 8 i (i < 8), of
+// the keys and of the values, so every load instruction reads whole rows of 8 lanes and all of them are in flight at
+// once, with no branch around them (this call's own entries and entries past the ring are read at a valid place and
+// replaced or masked after). A score is 8 products a lane and a sum over the row's 8 lanes (DPP); the lane then holds
+// the probability of exactly the value rows it holds, so nothing passes through LDS between softmax and P.V. Each wave
+// keeps its own maximum, sum and output over its 64 entries; the four meet in LDS: two barriers in all. One key row a
+// thread read whole took 62 us a layer at 224 seats (float32) against MEASURE_RA now: its loads touched 64 rows of
+// 2 KB pitch each, 16 bytes at a time, more lines than the L1 holds. STREAM: the rings of all layers and seats exceed
+// the 256 MB memory-side cache, so the rows are read with the non-temporal hint.
+// The head-0 workgroup records key_pos; every workgroup knows the positions of the entries this call writes, so none
+// depends on another's key_pos write.
 constexpr int RA_HD = 64;
 constexpr int RA_RING = 256;
 constexpr int RA_T = 2;  // tokens per call: Mimi's upsample makes 2 per frame
 static_assert(RA_T <= 4, "one wave of the 4-wave workgroup per token");
-template <int DT, int TM>
+// K and V bytes of one layer's call from which the rings of a codec's 8 layers pass the 256 MB memory-side cache
+constexpr long RA_STREAM_BYTES = 32L << 20;
+
+template <int DT, bool STREAM> __device__ __forceinline__ V8<DT> ld_ring(const Elt<DT>* p) {
+  if constexpr (!STREAM) {
+    return ldv<DT>(p);
+  } else if constexpr (DT == M3X_F32) {
+    f32x8 r;
+    const u16x8 a = ld16_nt((const uint16_t*)p), c = ld16_nt((const uint16_t*)(p + 4));
+    const float4 x = __builtin_bit_cast(float4, a), y = __builtin_bit_cast(float4, c);
+    r.v[0] = x.x, r.v[1] = x.y, r.v[2] = x.z, r.v[3] = x.w, r.v[4] = y.x, r.v[5] = y.y, r.v[6] = y.z, r.v[7] = y.w;
+    return r;
+  } else {
+    return ld16_nt(p);
+  }
+}
+
+template <int DT, int TM, bool STREAM>
 __global__ __launch_bounds__(256) void ring_attn_kernel(const Elt<DT>* __restrict__ qkv, long ld_qkv,
                                                         Elt<DT>* kring, Elt<DT>* vring, int64_t* key_pos,
                                                         const int64_t* __restrict__ tokens,
@@ -573,14 +596,13 @@ __global__ __launch_bounds__(256) void ring_attn_kernel(const Elt<DT>* __restric
                                                         const float* __restrict__ inv_freq, float rope_scale,
                                                         Elt<DT>* __restrict__ out, long ld_out, int T, int H, int ring,
                                                         int window) {
-  __shared__ float qs[TM][RA_HD];
-  __shared__ float pw[TM][RA_RING];
-  __shared__ float red[2][TM][4];
+  __shared__ __align__(16) float qs[TM][RA_HD];
+  __shared__ float wm[TM][4], wl[TM][4];
   __shared__ float part[4][TM][RA_HD];
   __shared__ __align__(16) Elt<DT> knew[TM][RA_HD];  // this call's keys (post-RoPE) and values, stored to the
   __shared__ __align__(16) Elt<DT> vnew[TM][RA_HD];  // ring only at the end: reads of them come from here
-  const int b = blockIdx.x, h = blockIdx.y;
-  const int tid = threadIdx.x, wave = tid >> 6, l = tid & 63;
+  const int b = blockIdx.x / H, h = blockIdx.x - b * H;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63;
   const long slot = slots[b];
   // wave w < T handles token w: its q, k, v elements do not depend on the position, so they load first
   const int half = RA_HD / 2;
@@ -599,30 +621,21 @@ __global__ __launch_bounds__(256) void ring_attn_kernel(const Elt<DT>* __restric
   Elt<DT>* kr = kring + slot * (long)ring * H * RA_HD;  // [ring][H][hd]
   Elt<DT>* vr = vring + slot * (long)ring * H * RA_HD;
   int64_t* kp = key_pos + slot * (long)ring;
-  const int lo = (int)(p0 % ring);  // ring entry of token 0; token t sits at (lo + t) % ring
-  // the older entries' keys, positions and values load now, while RoPE runs; this call's own rows come from LDS
-  // after the barrier. Thread j owns entry j for the scores; for P.V lane (g, d8) of wave w takes entries
-  // 64 w + g + 8 i, dims 8 d8 .. + 7.
-  const int j = tid;
-  const int dd = (j - lo + ring) % ring;  // entries this call writes hold p0 + dd, dd < T
-  long kj = NEVER_POS;
-  V8<DT> k8[RA_HD / 8];
-#pragma unroll
-  for (int d = 0; d < RA_HD / 8; ++d) k8[d] = zero_v8<DT>();
-  if (j < ring && dd >= T) {
-    const Elt<DT>* krow = kr + ((long)j * H + h) * RA_HD;
-#pragma unroll
-    for (int d = 0; d < RA_HD / 8; ++d) k8[d] = ldv<DT>(krow + 8 * d);
-    kj = kp[j];
-  }
   const int g = l >> 3, dc = 8 * (l & 7);
-  V8<DT> vv[8];
+  V8<DT> kk[8], vv[8];
+  long kj[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
-    const int jj = 64 * wave + g + 8 * i;
-    vv[i] = zero_v8<DT>();
-    if (jj < ring && (jj - lo + ring) % ring >= T) vv[i] = ldv<DT>(vr + ((long)jj * H + h) * RA_HD + dc);
+    const int jc = min(64 * wave + g + 8 * i, ring - 1);
+    kk[i] = ld_ring<DT, STREAM>(kr + ((long)jc * H + h) * RA_HD + dc);
+    kj[i] = kp[jc];
   }
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int jc = min(64 * wave + g + 8 * i, ring - 1);
+    vv[i] = ld_ring<DT, STREAM>(vr + ((long)jc * H + h) * RA_HD + dc);
+  }
+  const int lo = (int)(p0 % ring);  // ring entry of token 0; token t sits at (lo + t) % ring
   if (wave < T) {  // RoPE of token `wave`
     const float f = inv_freq[l < half ? l : l - half];
     const float sgn = l < half ? -1.f : 1.f;
@@ -633,93 +646,85 @@ __global__ __launch_bounds__(256) void ring_attn_kernel(const Elt<DT>* __restric
     vnew[wave][l] = v_l;
   }
   __syncthreads();  // queries and this call's rows are in LDS
-  if (j < ring && dd < T) {
-    kj = p0 + dd;
+  float q[TM][8];
 #pragma unroll
-    for (int d = 0; d < RA_HD / 8; ++d) k8[d] = *reinterpret_cast<const V8<DT>*>(&knew[dd][8 * d]);
+  for (int t = 0; t < TM; ++t) {
+    const float4 qa = *reinterpret_cast<const float4*>(&qs[t][dc]);
+    const float4 qb = *reinterpret_cast<const float4*>(&qs[t][dc + 4]);
+    q[t][0] = qa.x, q[t][1] = qa.y, q[t][2] = qa.z, q[t][3] = qa.w;
+    q[t][4] = qb.x, q[t][5] = qb.y, q[t][6] = qb.z, q[t][7] = qb.w;
   }
+  float s[TM][8], m[TM];
+#pragma unroll
+  for (int t = 0; t < TM; ++t) m[t] = -INFINITY;
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     const int jj = 64 * wave + g + 8 * i;
-    const int dn = (jj - lo + ring) % ring;
-    if (jj < ring && dn < T) vv[i] = *reinterpret_cast<const V8<DT>*>(&vnew[dn][dc]);
-  }
-  float sc[TM];
+    int dd = jj - lo;  // entries this call writes hold p0 + dd, dd < T
+    if (dd < 0) dd += ring;
+    const bool own = jj < ring && dd < T;
+    if (__ballot(own)) {  // at most T rows of the workgroup
+      const V8<DT> kn = *reinterpret_cast<const V8<DT>*>(&knew[own ? dd : 0][dc]);
+      const V8<DT> vn = *reinterpret_cast<const V8<DT>*>(&vnew[own ? dd : 0][dc]);
 #pragma unroll
-  for (int t = 0; t < TM; ++t) {
-    sc[t] = -INFINITY;
-    if (t >= T) continue;
-    float acc = 0.f;
-#pragma unroll
-    for (int d = 0; d < RA_HD / 8; ++d) {
-      const float4 qa = *reinterpret_cast<const float4*>(&qs[t][8 * d]);
-      const float4 qb = *reinterpret_cast<const float4*>(&qs[t][8 * d + 4]);
-      acc += qa.x * E<DT>::to_f(k8[d].v[0]) + qa.y * E<DT>::to_f(k8[d].v[1]) + qa.z * E<DT>::to_f(k8[d].v[2]) +
-             qa.w * E<DT>::to_f(k8[d].v[3]) + qb.x * E<DT>::to_f(k8[d].v[4]) + qb.y * E<DT>::to_f(k8[d].v[5]) +
-             qb.z * E<DT>::to_f(k8[d].v[6]) + qb.w * E<DT>::to_f(k8[d].v[7]);
+      for (int e = 0; e < 8; ++e) {
+        kk[i].v[e] = own ? kn.v[e] : kk[i].v[e];
+        vv[i].v[e] = own ? vn.v[e] : vv[i].v[e];
+      }
     }
-    const long pos = p0 + t;
-    if (kj <= pos && kj > pos - window) sc[t] = acc * 0.125f;  // NEVER_POS and j >= ring never qualify
-  }
-  // block-wide softmax per query
-#pragma unroll
-  for (int t = 0; t < TM; ++t) {
-    if (t >= T) break;
-    const float m = wave_max_xor(sc[t], 64);
-    if (l == 0) red[0][t][wave] = m;
-  }
-  __syncthreads();
-  float mx[TM];
-#pragma unroll
-  for (int t = 0; t < TM; ++t) {
-    if (t >= T) break;
-    mx[t] = fmaxf(fmaxf(red[0][t][0], red[0][t][1]), fmaxf(red[0][t][2], red[0][t][3]));  // finite: own key
-    const float pe = sc[t] == -INFINITY ? 0.f : expf(sc[t] - mx[t]);
-    if (j < ring) pw[t][j] = pe;
-    const float sm = wave_sum_xor(pe, 64);
-    if (l == 0) red[1][t][wave] = sm;
-  }
-  __syncthreads();
-  // P.V over this wave's 64 entries (values loaded above)
-  float o[TM][8];
-#pragma unroll
-  for (int t = 0; t < TM; ++t)
-#pragma unroll
-    for (int e = 0; e < 8; ++e) o[t][e] = 0.f;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int jj = 64 * wave + g + 8 * i;
+    const long pj = jj >= ring ? NEVER_POS : own ? p0 + dd : kj[i];
 #pragma unroll
     for (int t = 0; t < TM; ++t) {
-      if (t >= T) continue;
-      const float pj = jj < ring ? pw[t][jj] : 0.f;  // 0 for masked entries, whose values are finite
+      float acc = 0.f;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) o[t][e] += pj * E<DT>::to_f(vv[i].v[e]);
+      for (int e = 0; e < 8; ++e) acc = fmaf(q[t][e], E<DT>::to_f(kk[i].v[e]), acc);
+      acc = group_sum<8>(acc) * 0.125f;
+      const long pos = p0 + t;
+      s[t][i] = pj <= pos && pj > pos - window ? acc : -INFINITY;  // NEVER_POS never qualifies
+      m[t] = fmaxf(m[t], s[t][i]);
     }
   }
 #pragma unroll
   for (int t = 0; t < TM; ++t) {
     if (t >= T) break;
+    m[t] = across_max<8>(m[t]);
+    float sum = 0.f, o[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      float v = o[t][e];
-      v += __shfl_xor(v, 8, 64);
-      v += __shfl_xor(v, 16, 64);
-      v += __shfl_xor(v, 32, 64);
-      o[t][e] = v;
+    for (int e = 0; e < 8; ++e) o[e] = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      // masked rows weigh 0 (their values may be anything a stale ring row holds: finite, or never written)
+      const float p = s[t][i] == -INFINITY ? 0.f : expf(s[t][i] - m[t]);
+      sum += p;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) o[e] = fmaf(p, E<DT>::to_f(vv[i].v[e]), o[e]);
     }
-    if (g == 0) {
+    sum = across_sum<8>(sum);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) part[wave][t][dc + e] = o[t][e];
+    for (int e = 0; e < 8; ++e) o[e] = across_sum<8>(o[e]);
+    if (g == 0) {
+      float* pt = &part[wave][t][dc];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) pt[e] = o[e];
+    }
+    if (l == 0) {
+      wm[t][wave] = m[t];
+      wl[t][wave] = sum;
     }
   }
   __syncthreads();
   for (int i = tid; i < T * RA_HD; i += 256) {
     const int t = i / RA_HD, d = i % RA_HD;
-    const float sum = red[1][t][0] + red[1][t][1] + red[1][t][2] + red[1][t][3];
-    const float v = part[0][t][d] + part[1][t][d] + part[2][t][d] + part[3][t][d];
+    const float mx = fmaxf(fmaxf(wm[t][0], wm[t][1]), fmaxf(wm[t][2], wm[t][3]));  // finite: own key
+    float sum = 0.f, v = 0.f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const float f = wm[t][w] == -INFINITY ? 0.f : expf(wm[t][w] - mx);
+      sum = fmaf(f, wl[t][w], sum);
+      v = fmaf(f, part[w][t][d], v);
+    }
     out[((long)b * T + t) * ld_out + h * RA_HD + d] = E<DT>::from_f(v / sum);
-    // this call's rows into the ring (no thread of this workgroup reads them from global memory)
+    // this call's rows into the ring (every wave has read its rows of it)
     const long e = (lo + t) % ring;
     kr[(e * H + h) * RA_HD + d] = knew[t][d];
     vr[(e * H + h) * RA_HD + d] = vnew[t][d];
@@ -958,14 +963,22 @@ M3X_API int m3x_ring_attn(const void* qkv, long ld_qkv, void* kring, void* vring
   if (!qkv || !kring || !vring || !key_pos || !tokens || !slots || !inv_freq || !out) return M3X_ENULL;
   if (!m3x_aligned16(qkv) || !m3x_aligned16(kring)) return M3X_EINVAL;
   if (!m3x_aligned16(out) || (ld_out & 7)) return M3X_EINVAL;
-#define RA_LAUNCH(DTT, TMM)                                                                                    \
-  hipLaunchKernelGGL((ring_attn_kernel<DTT, TMM>), dim3(B, H), dim3(256), 0, (hipStream_t)stream,                  \
-                     (const Elt<DTT>*)qkv, ld_qkv, (Elt<DTT>*)kring, (Elt<DTT>*)vring, key_pos, tokens, slots,      \
+  if ((long)B * H > 0x7fffffffL) return M3X_EINVAL;
+  const bool stream_rows = (long)B * ring * H * RA_HD * 2 * (dtype == M3X_F32 ? 4 : 2) >= RA_STREAM_BYTES;
+#define RA_LAUNCH(DTT, STR)                                                                                       \
+  hipLaunchKernelGGL((ring_attn_kernel<DTT, RA_T, STR>), dim3((unsigned)(B * H)), dim3(256), 0, (hipStream_t)stream, \
+                     (const Elt<DTT>*)qkv, ld_qkv, (Elt<DTT>*)kring, (Elt<DTT>*)vring, key_pos, tokens, slots,        \
                      inv_freq, rope_scale, (Elt<DTT>*)out, ld_out, T, H, ring, window)
-  if (dtype == M3X_F16) RA_LAUNCH(M3X_F16, RA_T);
-  else if (dtype == M3X_BF16) RA_LAUNCH(M3X_BF16, RA_T);
-  else if (dtype == M3X_F32) RA_LAUNCH(M3X_F32, RA_T);
+#define RA_DT(DTT)                      \
+  do {                                  \
+    if (stream_rows) RA_LAUNCH(DTT, true); \
+    else RA_LAUNCH(DTT, false);         \
+  } while (0)
+  if (dtype == M3X_F16) RA_DT(M3X_F16);
+  else if (dtype == M3X_BF16) RA_DT(M3X_BF16);
+  else if (dtype == M3X_F32) RA_DT(M3X_F32);
   else return M3X_EUNSUPPORTED;
+#undef RA_DT
 #undef RA_LAUNCH
   M3X_CHECK_LAUNCH();
   return M3X_OK;
