@@ -10,7 +10,6 @@
 // most CODEC_KEEP state values across that barrier.
 constexpr int CODEC_THREADS = 256;
 constexpr int CODEC_KEEP = 16;
-constexpr long NEVER_POS = -(1L << 40);  // key_pos of an empty ring entry
 
 // ---------------------------------------------------------------------------------------------------------
 // RVQ decode (:134-149; transformers MimiSplitResidualVectorQuantizer.decode): out[b, :dim] = table_0[code_0]
@@ -562,7 +561,7 @@ __global__ __launch_bounds__(CODEC_THREADS) void convt_overlap_kernel(const Elt<
 // replaced or masked after). A score is 8 products a lane and a sum over the row's 8 lanes (DPP); the lane then holds
 // the probability of exactly the value rows it holds, so nothing passes through LDS between softmax and P.V. Each wave
 // keeps its own maximum, sum and output over its 64 entries; the four meet in LDS: two barriers in all. One key row a
-// thread read whole took 62 us a layer at 224 seats (float32) against MEASURE_RA now: its loads touched 64 rows of
+// thread read whole took 62 us a layer at 224 seats (float32) against 53 now: its loads touched 64 rows of
 // 2 KB pitch each, 16 bytes at a time, more lines than the L1 holds. STREAM: the rings of all layers and seats exceed
 // the 256 MB memory-side cache, so the rows are read with the non-temporal hint.
 // The head-0 workgroup records key_pos; every workgroup knows the positions of the entries this call writes, so none
@@ -589,7 +588,7 @@ template <int DT, bool STREAM> __device__ __forceinline__ V8<DT> ld_ring(const E
 }
 
 template <int DT, int TM, bool STREAM>
-__global__ __launch_bounds__(256) void ring_attn_kernel(const Elt<DT>* __restrict__ qkv, long ld_qkv,
+__global__ __launch_bounds__(256, STREAM && DT == M3X_F32 ? 3 : 1) void ring_attn_kernel(const Elt<DT>* __restrict__ qkv, long ld_qkv,
                                                         Elt<DT>* kring, Elt<DT>* vring, int64_t* key_pos,
                                                         const int64_t* __restrict__ tokens,
                                                         const int64_t* __restrict__ slots,
@@ -598,6 +597,7 @@ __global__ __launch_bounds__(256) void ring_attn_kernel(const Elt<DT>* __restric
                                                         int window) {
   __shared__ __align__(16) float qs[TM][RA_HD];
   __shared__ float wm[TM][4], wl[TM][4];
+  __shared__ int age[RA_RING];  // how many positions an entry lies before token 0 (negative: never visible)
   __shared__ float part[4][TM][RA_HD];
   __shared__ __align__(16) Elt<DT> knew[TM][RA_HD];  // this call's keys (post-RoPE) and values, stored to the
   __shared__ __align__(16) Elt<DT> vnew[TM][RA_HD];  // ring only at the end: reads of them come from here
@@ -623,17 +623,22 @@ __global__ __launch_bounds__(256) void ring_attn_kernel(const Elt<DT>* __restric
   int64_t* kp = key_pos + slot * (long)ring;
   const int g = l >> 3, dc = 8 * (l & 7);
   V8<DT> kk[8], vv[8];
-  long kj[8];
+  const long kj = kp[min(tid, ring - 1)];
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     const int jc = min(64 * wave + g + 8 * i, ring - 1);
     kk[i] = ld_ring<DT, STREAM>(kr + ((long)jc * H + h) * RA_HD + dc);
-    kj[i] = kp[jc];
   }
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
+  auto vload = [&](int i) {
     const int jc = min(64 * wave + g + 8 * i, ring - 1);
     vv[i] = ld_ring<DT, STREAM>(vr + ((long)jc * H + h) * RA_HD + dc);
+  };
+  // every load at once, one round trip; float32 streaming: a row's values take the registers of its consumed keys,
+  // so that three workgroups a CU fit instead of two
+  constexpr bool LATE = STREAM && DT == M3X_F32;
+  if constexpr (!LATE) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) vload(i);
   }
   const int lo = (int)(p0 % ring);  // ring entry of token 0; token t sits at (lo + t) % ring
   if (wave < T) {  // RoPE of token `wave`
@@ -645,7 +650,13 @@ __global__ __launch_bounds__(256) void ring_attn_kernel(const Elt<DT>* __restric
     knew[wave][l] = E<DT>::from_f(k_l * cs + sgn * k_p * sn);
     vnew[wave][l] = v_l;
   }
-  __syncthreads();  // queries and this call's rows are in LDS
+  {
+    int dd = tid - lo;  // entries this call writes hold p0 + dd, dd < T
+    if (dd < 0) dd += ring;
+    // an older entry outside (p0 - window, p0) is never visible; window <= ring, so an age fits an int
+    age[tid] = tid >= ring ? RA_RING : dd < T ? -dd : kj > p0 - window && kj < p0 ? (int)(p0 - kj) : RA_RING;
+  }
+  __syncthreads();  // queries, this call's rows and the ages are in LDS
   float q[TM][8];
 #pragma unroll
   for (int t = 0; t < TM; ++t) {
@@ -663,25 +674,27 @@ __global__ __launch_bounds__(256) void ring_attn_kernel(const Elt<DT>* __restric
     int dd = jj - lo;  // entries this call writes hold p0 + dd, dd < T
     if (dd < 0) dd += ring;
     const bool own = jj < ring && dd < T;
-    if (__ballot(own)) {  // at most T rows of the workgroup
+    const bool any_own = __ballot(own) != 0;  // at most T rows of the workgroup
+    if (any_own) {
       const V8<DT> kn = *reinterpret_cast<const V8<DT>*>(&knew[own ? dd : 0][dc]);
-      const V8<DT> vn = *reinterpret_cast<const V8<DT>*>(&vnew[own ? dd : 0][dc]);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        kk[i].v[e] = own ? kn.v[e] : kk[i].v[e];
-        vv[i].v[e] = own ? vn.v[e] : vv[i].v[e];
-      }
+      for (int e = 0; e < 8; ++e) kk[i].v[e] = own ? kn.v[e] : kk[i].v[e];
     }
-    const long pj = jj >= ring ? NEVER_POS : own ? p0 + dd : kj[i];
+    const int aj = age[jj];
 #pragma unroll
     for (int t = 0; t < TM; ++t) {
       float acc = 0.f;
 #pragma unroll
       for (int e = 0; e < 8; ++e) acc = fmaf(q[t][e], E<DT>::to_f(kk[i].v[e]), acc);
       acc = group_sum<8>(acc) * 0.125f;
-      const long pos = p0 + t;
-      s[t][i] = pj <= pos && pj > pos - window ? acc : -INFINITY;  // NEVER_POS never qualifies
+      s[t][i] = aj + t >= 0 && aj + t < window ? acc : -INFINITY;  // token t: p0 + t - window < position <= p0 + t
       m[t] = fmaxf(m[t], s[t][i]);
+    }
+    if constexpr (LATE) vload(i);
+    if (any_own) {
+      const V8<DT> vn = *reinterpret_cast<const V8<DT>*>(&vnew[own ? dd : 0][dc]);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) vv[i].v[e] = own ? vn.v[e] : vv[i].v[e];
     }
   }
 #pragma unroll
