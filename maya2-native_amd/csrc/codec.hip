@@ -157,6 +157,7 @@ __global__ __launch_bounds__(256) void resid_ln_kernel(Elt<DT>* h, long ld_h, co
   if (row >= rows) return;  // a whole wave; the kernel has no block barrier
   const int c = 8 * (threadIdx.x & 63);
   const V8<DT> hv = ldv<DT>(h + row * ld_h + c), av = ldv<DT>(a + row * ld_a + c), sv = ldv<DT>(scale + c);
+  const V8<DT> wv = ldv<DT>(w + c), bv = ldv<DT>(b + c);  // one round trip for every operand
   float v[8];
   V8<DT> ho;
   float sum = 0.f;
@@ -169,15 +170,14 @@ __global__ __launch_bounds__(256) void resid_ln_kernel(Elt<DT>* h, long ld_h, co
     sum += v[e];
   }
   stv<DT>(h + row * ld_h + c, ho);
-  const float mean = wave_sum_xor(sum, 64) / (float)RLN_N;
+  const float mean = xor32_sum(xor16_sum(group_sum<16>(sum))) / (float)RLN_N;
   float sq = 0.f;
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
     v[e] = v[e] - mean;
     sq += v[e] * v[e];
   }
-  const float inv = 1.f / sqrtf(wave_sum_xor(sq, 64) / (float)RLN_N + eps);
-  const V8<DT> wv = ldv<DT>(w + c), bv = ldv<DT>(b + c);
+  const float inv = 1.f / sqrtf(xor32_sum(xor16_sum(group_sum<16>(sq))) / (float)RLN_N + eps);
   V8<DT> yo;
 #pragma unroll
   for (int e = 0; e < 8; ++e) yo.v[e] = E<DT>::from_f(v[e] * inv * E<DT>::to_f(wv.v[e]) + E<DT>::to_f(bv.v[e]));
@@ -347,7 +347,11 @@ __global__ __launch_bounds__(256) void conv_gemm_kernel(const Elt<DT>* __restric
 // all taps from LDS: a tap's fragment is the same rows shifted by tap * dil (row r sits in slot r % 16, XOR-swizzled by
 // its k group, of fragment r / 16, so 16 consecutive rows hit 16 bank groups wherever they start). The products add up
 // channel block by channel block, taps within.
+// 224 seats (MI355X, inside the frame, conv_gemm_kernel against it): 64 -> 32 channels of 1920 rows a seat 128 / 70 us,
+// 128 -> 64 of 480 108 / 58, 256 -> 128 of 96 112 / 46. One seat: 4 workgroups 16.6 / 25.7 us, 15 workgroups 10.2 / 12.9, so
+// it takes CX_MIN_BLOCKS of them.
 constexpr int CX_ROWS = 128, CX_PAD = 16;  // rows a workgroup, most history frames
+constexpr long CX_MIN_BLOCKS = 160;
 
 template <int CT, int TAPS>
 __global__ __launch_bounds__(256) void conv_x3_kernel(const float* __restrict__ X, long ldx,
@@ -1073,10 +1077,10 @@ M3X_API int m3x_conv_gemm(const void* x, long ldx, const void* w_packed, const v
     const F32Epi ep{(const float*)bias, (const float*)res, ld_res, use_elu};
     const float *X = (const float*)x, *W = (const float*)w_packed;
     // conv_x3_kernel: whole channel blocks, 3 taps, 32 or 64 columns a workgroup, at least 70 % of its 128-row blocks'
-    // rows live, enough workgroups for the chip; reads of x overlapping its own output (y = x in place) are out
+    // rows live, enough workgroups; reads of x overlapping its own output (y = x in place) are out
     const int rblk = G ? m3x_ceil_div(T, CX_ROWS) : 0, ncol = N == 32 ? 32 : 64;
     if (G && C % 32 == 0 && K == 3 * C && cs.pad <= CX_PAD && N >= 32 && 10L * T >= 7L * rblk * CX_ROWS && y != x &&
-        (long)(M / T) * rblk * (N / ncol) >= F32X3_MIN_BLOCKS) {
+        (long)(M / T) * rblk * (N / ncol) >= CX_MIN_BLOCKS && (long)(M / T) * rblk <= 0x7fffffffL) {
       const dim3 gx3((unsigned)((long)(M / T) * rblk), N / ncol);
       if (ncol == 32)
         hipLaunchKernelGGL((conv_x3_kernel<2, 3>), gx3, dim3(256), 0, st, X, ldx, W, (float*)y, ldy, rblk, ep, cs);

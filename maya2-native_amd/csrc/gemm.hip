@@ -202,6 +202,49 @@ __global__ __launch_bounds__(256) void linear_f32_kernel(const float* __restrict
   }
 }
 
+// fp32 projections of up to 16 rows (a few Mimi seats): one workgroup of 16 waves per weight tile, a sixteenth of K each.
+// A wave loads its S weight fragments and the matching activations (straight into the B operand; rows past M repeat
+// row M - 1) at once, so the kernel pays one memory round trip however long K is; the 16 partial tiles meet in LDS and
+// are added in slice order. Against 4 waves walking chunks of 4 steps (MI355X, weights not in L2, us): 2 x 512 x 512 3.5 ->
+// 2.8, 2 x 512 x 2048 7.6 -> 5.6, 2 x 1024 x 3584 13.3 -> 9.9, 2 x 8192 x 1024 13.0 -> 7.8, 16 x 512 x 2048 8.2 -> 7.2. Bound by
+// the launch and by what one CU streams from behind its L2 (~25 GB/s: 128 KB a workgroup at K = 2048).
+template <int S, int EPI>
+__global__ __launch_bounds__(1024) void linear_f32_rows_kernel(const float* __restrict__ X, long ldx,
+                                                               const float* __restrict__ Wp, float* __restrict__ Y,
+                                                               long ldy, int M, int N, int K) {
+  __shared__ __align__(16) float red[16][256];
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63;
+  const int li = lane & 15;
+  const int lg = lane >> 4;
+  const int ksteps = K >> 5;
+  const int span = (ksteps + 15) >> 4;  // steps a wave, <= S
+  const int s0 = wave * span;
+  const float* xp = X + (long)min(li, M - 1) * ldx + 8 * lg;
+  const float* wp = Wp + (long)blockIdx.x * ksteps * 512 + 8 * lane;
+  f32x8 w[S], x[S];
+#pragma unroll
+  for (int i = 0; i < S; ++i) {  // steps past the slice or K: a valid fragment, never multiplied
+    const int s = min(s0 + min(i, span - 1), ksteps - 1);
+    x[i] = ldv<M3X_F32>(xp + s * 32);
+    w[i] = ldv<M3X_F32>(wp + (long)s * 512);
+  }
+  f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < S; ++i)
+    if (i < span && s0 + i < ksteps) acc = mfma16x16x32_f32(w[i], x[i], acc);  // wave-uniform
+  *reinterpret_cast<f32x4_t*>(&red[wave][16 * li + 4 * lg]) = acc;
+  __syncthreads();
+  if (tid >= 256) return;
+  const int m = tid >> 4, n = blockIdx.x * 16 + (tid & 15);
+  float v = red[0][tid];
+#pragma unroll
+  for (int q = 1; q < 16; ++q) v = v + red[q][tid];
+  if constexpr (EPI == EPI_GELU) v = 0.5f * v * (1.0f + erff(v * 0.70710678118654752f));
+  if (m < M && n < N) Y[(long)m * ldy + n] = v;
+}
+
 // fp32 tile choice. From F32X3_MIN_BLOCKS workgroups of 64 x 64 (rows beyond one 32-row block) the plain and GELU
 // projections take linear_f32x3_kernel, which has no K split and needs the chip filled: with weights that the launch
 // before did not leave in the caches, 448 x 2048 x 512 (224 workgroups) took 19.4 us against 16.1 and 448 x 1536 x 512
@@ -212,12 +255,24 @@ __global__ __launch_bounds__(256) void linear_f32_kernel(const float* __restrict
 // SwiGLU, the fp32 instructions: the largest tile (most operand reuse) that still gives at least 256 workgroups; small
 // grids split K four ways.
 constexpr long F32X3_WIDE_BLOCKS = 440;
+constexpr int ROWS_MAX_TILES = 1024;  // workgroups of linear_f32_rows_kernel; more columns keep the chip busy in any form
 
 template <int EPI>
 static bool launch_linear_f32(hipStream_t st, const float* X, long ldx, const float* W, const float* W2, float* Y,
                               long ldy, int M, int N, int K) {
   const int ntiles = m3x_ceil_div(N, 16);
   if constexpr (EPI != EPI_SWIGLU) {
+    if (M <= 16 && K <= 4096 && ntiles <= ROWS_MAX_TILES) {
+#define M3X_LR(SS) \
+  hipLaunchKernelGGL((linear_f32_rows_kernel<SS, EPI>), dim3(ntiles), dim3(1024), 0, st, X, ldx, W, Y, ldy, M, N, K)
+      const int span = m3x_ceil_div(K, 512);
+      if (span <= 1) M3X_LR(1);
+      else if (span <= 2) M3X_LR(2);
+      else if (span <= 4) M3X_LR(4);
+      else M3X_LR(8);
+#undef M3X_LR
+      return true;
+    }
     const int mblk = m3x_ceil_div(M, 64), nblk = m3x_ceil_div(N, 64), nwide = m3x_ceil_div(N, 128);
     const F32Epi ep{};
     if (M > 32 && (long)mblk * nblk >= F32X3_MIN_BLOCKS) {
@@ -234,6 +289,8 @@ static bool launch_linear_f32(hipStream_t st, const float* X, long ldx, const fl
   const int cand[6][2] = {{4, 4}, {2, 4}, {2, 2}, {1, 4}, {1, 2}, {1, 1}};
   int mt = 1, nw = 1;
   for (const auto& c : cand) {
+    // 256 tiles of 64 x 64 take the kernel above, unless of 32 rows or fewer, for which 64-row tiles are half empty
+    if (EPI != EPI_SWIGLU && c[0] == 4) continue;
     if ((long)m3x_ceil_div(M, 16 * c[0]) * m3x_ceil_div(ntiles, c[1]) >= 256) {
       mt = c[0];
       nw = c[1];
@@ -248,8 +305,8 @@ static bool launch_linear_f32(hipStream_t st, const float* X, long ldx, const fl
                      mblk, nblk)
   switch (mt * 10 + nw) {
     case 44:
-      if constexpr (EPI == EPI_SWIGLU) M3X_LF(4, 4);  // 256 such tiles of the others take the kernel above
-      return EPI == EPI_SWIGLU;
+      if constexpr (EPI == EPI_SWIGLU) M3X_LF(4, 4);
+      return true;
     case 24: M3X_LF(2, 4); return true;
     case 22: M3X_LF(2, 2); return true;
     case 14: M3X_LF(1, 4); return true;

@@ -40,6 +40,27 @@ def test_linear_f32x3(gpu, M, N, K, gelu):
     assert bool(((y.double() - ref).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("M", [1, 2, 15, 16, 17])
+@pytest.mark.parametrize("N,K", [(512, 512), (100, 32), (1537, 96), (512, 2048), (64, 4096), (48, 3584), (16400, 64),
+                                 (33, 4128)])
+@pytest.mark.parametrize("gelu", [False, True])
+def test_linear_f32_few_rows(gpu, M, N, K, gelu):
+    """Up to 16 rows: one workgroup of 16 K slices per tile (K up to 4096, up to 1024 tiles)."""
+    from m3x import ops
+    g = _g(M + N + K)
+    x = torch.randn(M, K, generator=g).to(gpu)
+    w = (torch.randn(N, K, generator=g) * K ** -0.5).to(gpu)
+    y = torch.full((M + 1, N), 7.0, device=gpu)
+    pw = ops.pack_weight(w)
+    ops.linear_act(x, pw, None, ops.ACT_GELU, y[:M]) if gelu else ops.linear(x, pw, y[:M])
+    ref = x.double() @ w.double().t()
+    bound = (K / 4 + 20) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())  # K / 4 additions and the slices'
+    if gelu:
+        ref = F.gelu(ref)
+        bound = 1.13 * bound + 2.0 ** -21 * ref.abs() + 2.0 ** -22
+    assert bool(((y[:M].double() - ref).abs() <= bound).all()) and bool((y[M] == 7.0).all())
+
+
 def test_linear_f32x3_nonfinite(gpu):
     """Rows with infinities, NaN or values that bf16 rounds to infinity get what fp32 products give; the others are as
     without them."""
@@ -63,7 +84,7 @@ def test_linear_f32x3_nonfinite(gpu):
                                              (40, 480, 128, 64, 1, True), (100, 128, 32, 128, 8, False),
                                              (161, 97, 64, 32, 3, True), (20, 1000, 32, 64, 1, False),
                                              (90, 130, 32, 64, 1, True),  # half-empty row blocks: the fp32 kernel
-                                             (7, 96, 64, 64, 1, True)])   # few workgroups: the fp32 kernel
+                                             (7, 96, 64, 64, 1, True), (1, 1920, 64, 32, 1, True)])  # few workgroups
 def test_conv_gemm_f32_gathered(gpu, B, T, C, N, dil, pre):
     from m3x import ops
     g = _g(B + T + C + N)
