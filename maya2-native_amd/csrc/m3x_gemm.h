@@ -1256,7 +1256,11 @@ static bool launch_linear(const LinearPlan& p, hipStream_t st, const uint16_t* X
                           const uint16_t* W2, uint16_t* Y, long ldy, int M, int N, int K, const NormIn& ni = NormIn{},
                           const ResidOut& ro = ResidOut{}, const QkOut& qk = QkOut{}) {
   static_assert(!(PRO && EPI == EPI_RESID), "a residual projection takes its input as is");
-  const StripTile t = strip_tile<EPI>(M, N, K, ldx);
+  // up to 512 rows a folded norm's statistics delay the strips' first stage: 416 x 3072 x 1024 inside the depth frame 16.4
+  // (plain) and 17.5 us (GELU) against 13.0 and 14.2 with the chunked plan, SwiGLU even. The bf16 q|k|v stays on the
+  // strips with its fused epilogue, and the plain product with it (same bits).
+  constexpr bool CHUNKED = PRO && !(DT == M3X_BF16 && (EPI == EPI_QKR || EPI == EPI_NONE));
+  const StripTile t = CHUNKED && M <= 512 ? StripTile{0, 0} : strip_tile<EPI>(M, N, K, ldx);
   if (t.rt) {
     const int nblk = m3x_ceil_div(N, 64 * t.ng), mblk = m3x_ceil_div(M, 16 * t.rt);
 #define M3X_STRIP(RTT, NGG)                                                                                           \
