@@ -240,10 +240,10 @@ __device__ bool hist_marks(const float (&x)[NE], int V, int k, float m, SM& sm, 
 // k = 50 of 2048. It needs no atomics and one barrier, whatever the shape of the row; a histogram of the distances below
 // the maximum serialised its atomics on a peaked row, whose bulk falls into a few bins. Rows of 2048 with one code 16
 // above the bulk, MI355X: the 224-seat depth frame (30 such samplers) 5.11 -> 4.94 ms, the one-seat frame 2.35 ->
-// 2.21 ms; head and codebook-0 sampler of 224 flat rows 24.2 -> 21.4 us. Larger k takes the histogram: the maxima would
-// let through several times k candidates (k = 200 of 2048: about 350). More than 256 candidates (an order that gathers
-// the leaders in a few threads, many repeats), or fewer than k threads with a maximum above -inf, take the exact radix
-// select.
+// 2.21 ms; head and codebook-0 sampler of 224 flat rows 24.2 -> 21.4 and 24.5 -> 22.8 us in two runs (repeats of one
+// build differ by 7 to 14 % there). Larger k takes the histogram: the maxima would let through several times k candidates
+// (k = 200 of 2048: about 350). More than 256 candidates (an order that gathers the leaders in a few threads, many
+// repeats), or fewer than k threads with a maximum above -inf, take the exact radix select.
 // The kernel runs every line of code once or twice a launch, so it is bound by latencies (dependent operations, barriers,
 // instruction fetch) and short loops beat unrolled code.
 constexpr int KFAST = 128;
