@@ -439,28 +439,22 @@ __global__ __launch_bounds__(256) void conv_x3_kernel(const float* __restrict__ 
       }
     }
   }
-  if (any_nonfinite<CT, RT>(acc)) {
+  if (wave > lastw) return;  // rows past T, never stored (no barrier follows)
 #pragma unroll
-    for (int a = 0; a < CT; ++a)
+  for (int a = 0; a < CT; ++a)
+    redo_unsure<RT>(
+        acc[a], n0 + 16 * a, n0 + 16 * CT, ks, [&](int s) { return ldv<M3X_F32>(wb + ((long)a * ks + s) * 512); },
+        [&](int s, int t) {
+          const int tap = s / cst;
+          const int i = t0 + min(16 * (wave * RT + t) + li + tap * cs.dil, rows - 1);
+          const int c = 32 * (s - tap * cst) + 8 * lg;
+          f32x8 x = ldv<M3X_F32>(i < cs.pad ? hs + (long)i * cs.C + c : xs + (long)i * ldx + c);
+          if (cs.pre_elu && i >= cs.pad) {
 #pragma unroll
-      for (int t = 0; t < RT; ++t) acc[a][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    for (int s = 0; s < ks; ++s) {
-      const int tap = s / cst;
-#pragma unroll
-      for (int t = 0; t < RT; ++t) {
-        const int i = t0 + min(16 * (wave * RT + t) + li + tap * cs.dil, rows - 1);
-        const int c = 32 * (s - tap * cst) + 8 * lg;
-        f32x8 x = ldv<M3X_F32>(i < cs.pad ? hs + (long)i * cs.C + c : xs + (long)i * ldx + c);
-        if (cs.pre_elu && i >= cs.pad) {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) x.v[e] = elu<M3X_F32>(x.v[e]);
-        }
-#pragma unroll
-        for (int a = 0; a < CT; ++a)
-          acc[a][t] = mfma16x16x32_f32(ldv<M3X_F32>(wb + ((long)a * ks + s) * 512), x, acc[a][t]);
-      }
-    }
-  }
+            for (int e = 0; e < 8; ++e) x.v[e] = elu<M3X_F32>(x.v[e]);
+          }
+          return x;
+        });
 #pragma unroll
   for (int t = 0; t < RT; ++t) {
     const int tr = t0 + 16 * (wave * RT + t) + li;

@@ -41,8 +41,8 @@ struct F32Epi {
 //
 // EPI 2 is m3x_conv_gemm's epilogue: bias, shortcut and ELU on the accumulators.
 //
-// A result that is not finite (an infinity or NaN in the operands, or a value that bf16(x) rounds to infinity) cannot
-// come out of the split sums as fp32 would give it: a wave that sees one redoes its tile on the fp32 instructions.
+// A result that is not finite (an infinity or NaN in the operands, or a value that bf16(x) rounds to infinity) cannot come
+// out of the split sums as fp32 would give it: such elements are taken from the fp32 instructions, one by one (redo_unsure).
 __device__ __forceinline__ void split_bf16x3(const f32x8& x, u16x8& h, u16x8& m, u16x8& l) {
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
@@ -65,17 +65,32 @@ __device__ __forceinline__ void mfma_x3(const u16x8 (&w)[3], const u16x8 (&b)[RT
     for (int t = 0; t < RT; ++t) acc[t] = mfma16x16x32<M3X_BF16>(w[PW[i]], b[t][PX[i]], acc[t]);
 }
 
-// Whether any of the wave's accumulators is infinite or NaN (its difference to itself is not 0); wave-uniform.
-template <int CT, int RT>
-__device__ __forceinline__ bool any_nonfinite(const f32x4_t (&acc)[CT][RT]) {
-  float bad = 0.f;
+// Whether a split sum is not what fp32 would give: it is infinite or NaN.
+__device__ __forceinline__ bool split_unsure(float v) { return (__float_as_uint(v) & 0x7f800000u) == 0x7f800000u; }
+
+// Such elements of a weight tile's RT row tiles, taken from the fp32 instructions (wt(s), xt(s, t): the fragments of k step s);
+// the others keep their sums, so that an element depends on its own row and column alone. Called by a whole wave.
+template <int RT, class WT, class XT>
+__device__ __forceinline__ void redo_unsure(f32x4_t (&acc)[RT], int n, int N, int ksteps, WT wt, XT xt) {
+  bool unsure = false;
 #pragma unroll
-  for (int a = 0; a < CT; ++a)
+  for (int t = 0; t < RT; ++t)
 #pragma unroll
-    for (int t = 0; t < RT; ++t)
+    for (int r = 0; r < 4; ++r) unsure |= n + r < N && split_unsure(acc[t][r]);
+  if (!__ballot(unsure)) return;
+  f32x4_t f[RT];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) bad += acc[a][t][r] - acc[a][t][r];
-  return __ballot(!(bad == 0.f)) != 0;
+  for (int t = 0; t < RT; ++t) f[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+  for (int s = 0; s < ksteps; ++s) {
+    const f32x8 w = wt(s);
+#pragma unroll
+    for (int t = 0; t < RT; ++t) f[t] = mfma16x16x32_f32(w, xt(s, t), f[t]);
+  }
+#pragma unroll
+  for (int t = 0; t < RT; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) acc[t][r] = split_unsure(acc[t][r]) ? f[t][r] : acc[t][r];
 }
 
 template <int WR, int RT, int CT, int EPI>  // EPI 0: plain, 1: GELU, 2: the conv epilogue
@@ -153,23 +168,15 @@ __global__ __launch_bounds__(256) void linear_f32x3_kernel(const float* __restri
     }
   }
 
-  if (any_nonfinite<CT, RT>(acc)) {
 #pragma unroll
-    for (int a = 0; a < CT; ++a)
-#pragma unroll
-      for (int t = 0; t < RT; ++t) acc[a][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    for (int s = 0; s < ksteps; ++s) {
-#pragma unroll
-      for (int a = 0; a < CT; ++a) {
-        const f32x8 w = ldv<M3X_F32>(Wp + ((long)min(t0 + wc * CT + a, ntiles - 1) * ksteps + s) * 512 + lane * 8);
-#pragma unroll
-        for (int t = 0; t < RT; ++t) {
-          const f32x8 x =
-              ldv<M3X_F32>(X + (long)min(m0 + 16 * (wr * RT + t) + li, M - 1) * ldx + s * 32 + 8 * lg);
-          acc[a][t] = mfma16x16x32_f32(w, x, acc[a][t]);
-        }
-      }
-    }
+  for (int a = 0; a < CT; ++a) {
+    const int tile = t0 + wc * CT + a;
+    redo_unsure<RT>(
+        acc[a], 16 * tile + 4 * lg, N, ksteps,
+        [&](int s) { return ldv<M3X_F32>(Wp + ((long)min(tile, ntiles - 1) * ksteps + s) * 512 + lane * 8); },
+        [&](int s, int t) {
+          return ldv<M3X_F32>(X + (long)min(m0 + 16 * (wr * RT + t) + li, M - 1) * ldx + s * 32 + 8 * lg);
+        });
   }
 
   const bool vec = (ldy & 3) == 0 && (((uintptr_t)Y) & 15) == 0;

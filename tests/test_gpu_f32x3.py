@@ -19,7 +19,9 @@ def _g(seed):
 
 
 @pytest.mark.parametrize("M,N,K", [(64, 10240, 64), (65, 5120, 32), (2500, 257, 96), (10304, 64, 64), (3000, 330, 160),
-                                   (33, 10300, 64), (14080, 128, 32), (28200, 100, 32), (127, 5120, 512)])
+                                   (33, 10300, 64), (14080, 128, 32), (28200, 100, 32), (127, 5120, 512),
+                                   (33, 16330, 32), (64, 16384, 64), (65, 8190, 96), (2500, 387, 96), (16321, 64, 64),
+                                   (64, 16320, 64)])  # 256 workgroups of 64 x 64, and 255
 @pytest.mark.parametrize("gelu", [False, True])
 def test_linear_f32x3(gpu, M, N, K, gelu):
     from m3x import ops
@@ -104,7 +106,8 @@ def test_conv_gemm_f32_gathered(gpu, B, T, C, N, dil, pre):
     assert bool(((y.double() - F.elu(pre_act)).abs() <= bound).all())
 
 
-@pytest.mark.parametrize("M,N,K", [(10240, 64, 32), (10303, 64, 96), (5130, 128, 64), (16000, 128, 32)])
+@pytest.mark.parametrize("M,N,K", [(10240, 64, 32), (10303, 64, 96), (5130, 128, 64), (16000, 128, 32), (16321, 64, 96),
+                                   (16320, 64, 96), (8130, 128, 64)])
 def test_conv_gemm_f32_plain(gpu, M, N, K):
     from m3x import ops
     g = _g(M + N + K)
@@ -115,3 +118,47 @@ def test_conv_gemm_f32_plain(gpu, M, N, K):
     bound = _bound(x.double().abs() @ w.double().abs().t() + bias.double().abs() + y.double().abs(), K, 10) + 2.0 ** -22
     ops.conv_gemm(x, ops.pack_weight(w), y, bias=bias, res=y, use_elu=True)
     assert bool(((y.double() - F.elu(ref)).abs() <= bound).all())
+
+
+def _conv_case(B, seed):
+    T, C, N = 96, 64, 64
+    g = _g(seed)
+    return (T, C, N, torch.randn(B * T, C, generator=g), torch.randn(B, 2 * C, generator=g),
+            torch.randn(N, 3 * C, generator=g) * (3 * C) ** -0.5)
+
+
+def test_nonfinite_rows_leave_the_others_alone(gpu):
+    """A row with infinities, NaN or values that bf16 rounds to infinity (a stream that broke) does not change a bit of the
+    other rows' (the other streams') results, in the projections, the plain conv and the gathered one."""
+    from m3x import ops
+    bad = torch.tensor([3, 70, 131, 200, 201, 699])
+    g = _g(6)
+    M, N, K = 700, 2048, 96
+    x = torch.randn(M, K, generator=g)
+    y = x.clone()
+    y[bad, 5] = torch.tensor([float("inf"), float("-inf"), float("nan"), 3.4e38, -3.4e38, float("nan")])
+    pw = ops.pack_weight(torch.randn(N, K, generator=g).to(gpu))
+    rows = torch.ones(M, dtype=torch.bool)
+    rows[bad] = False
+    a, b = ops.linear(x.to(gpu), pw), ops.linear(y.to(gpu), pw)
+    assert torch.equal(a[rows], b[rows])
+    assert bool(b[3].isinf().all()) and bool(b[70].isinf().all()) and bool(b[131].isnan().all()) and bool(b[699].isnan().all())
+    M = 16390
+    x = torch.randn(M, 64, generator=g)
+    y = x.clone()
+    y[bad + 9000, 1] = float("nan")
+    rows = torch.ones(M, dtype=torch.bool)
+    rows[bad + 9000] = False
+    pw = ops.pack_weight(torch.randn(64, 64, generator=g).to(gpu))
+    a, b = (ops.conv_gemm(t.to(gpu), pw, torch.empty(M, 64, device=gpu)) for t in (x, y))
+    assert torch.equal(a[rows], b[rows])
+    B = 160
+    T, C, N, x, state, w = _conv_case(B, 7)
+    y, state_y = x.clone().view(B, T, C), state.clone()
+    y[5, 40], y[17, 0], state_y[23] = float("nan"), float("inf"), float("nan")
+    pw, slots = ops.pack_weight(w.to(gpu)), torch.arange(B, device=gpu)
+    a, b = (ops.conv_gemm(t.reshape(B * T, C).to(gpu), pw, torch.empty(B * T, N, device=gpu),
+                          gather=(s.to(gpu), slots, T, C, 1, True)).view(B, T, N) for t, s in ((x, state), (y, state_y)))
+    clean = torch.ones(B, T, dtype=torch.bool)
+    clean[5, 40:43] = clean[17, :3] = clean[23, :2] = False  # a row's three taps
+    assert torch.equal(a[clean], b[clean]) and not bool(b[~clean].isfinite().all(1).any())
