@@ -22,12 +22,13 @@ struct F32Epi {
   int use_elu;
 };
 
-// fp32 projections on the bf16 matrix cores. Each fp32 operand is the exact sum of three bf16 values, h = bf16(x),
-// m = bf16(x - h), l = bf16(x - h - m) (8 significant bits each, 24 in all), and x . w is summed as
+// fp32 projections on the bf16 matrix cores. Each fp32 operand is the sum of three bf16 values, h = bf16(x),
+// m = bf16(x - h), l = bf16(x - h - m) (8 significant bits each, 24 in all; exact from 2^-110 up, within 2^-134 below, where l
+// and then m fall under bf16's smallest step), and x . w is summed as
 // l_x h_w + h_x l_w + m_x m_w + m_x h_w + h_x m_w + h_x h_w in fp32, smallest terms first: six
 // v_mfma_f32_16x16x32_bf16 a 16 x 16 x 32 step in place of eight v_mfma_f32_16x16x4_f32, 108 cycles instead of 259. The
-// products left out (m l, l m, l l) are below 2^-26 of the whole, under fp32's own rounding, and the accumulators round
-// once per 32 products instead of once per 4: against 64 bits the relative error of a product of N(0, 1) rows is
+// products left out (m l, l m, l l) are below 2^-25 of the whole, and the accumulators round six times per 32 products
+// instead of eight: against 64 bits the relative error of a product of N(0, 1) rows is
 // 2.3e-7 at K = 256 and 9.3e-7 at K = 3584, where the fp32 instructions give 2.9e-7 and 1.07e-6 (MI355X; about the
 // same for ELU outputs, lower for rows with an offset).
 //
@@ -41,8 +42,10 @@ struct F32Epi {
 //
 // EPI 2 is m3x_conv_gemm's epilogue: bias, shortcut and ELU on the accumulators.
 //
-// A result that is not finite (an infinity or NaN in the operands, or a value that bf16(x) rounds to infinity) cannot come
-// out of the split sums as fp32 would give it: such elements are taken from the fp32 instructions, one by one (redo_unsure).
+// Results that the split cannot give as fp32 would are taken from the fp32 instructions, element by element (redo_unsure):
+// those that are not finite (an infinity or NaN in the operands, or a value that bf16(x) rounds to infinity), and those
+// below 2^-48, where what the split loses of operands below 2^-110 (up to 2^-134 times the other operand's sum) may be more
+// than fp32's rounding. Before, x of 2^-126 N(0, 1) came out 2e-3 off and x of 2^-136 N(0, 1) as zeros, 2.9e-7 and 3.5e-5 in fp32.
 __device__ __forceinline__ void split_bf16x3(const f32x8& x, u16x8& h, u16x8& m, u16x8& l) {
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
@@ -65,32 +68,65 @@ __device__ __forceinline__ void mfma_x3(const u16x8 (&w)[3], const u16x8 (&b)[RT
     for (int t = 0; t < RT; ++t) acc[t] = mfma16x16x32<M3X_BF16>(w[PW[i]], b[t][PX[i]], acc[t]);
 }
 
-// Whether a split sum is not what fp32 would give: it is infinite or NaN.
-__device__ __forceinline__ bool split_unsure(float v) { return (__float_as_uint(v) & 0x7f800000u) == 0x7f800000u; }
+// Whether a split sum may be worse than fp32's: it is not finite, or below 2^-48 (zero included).
+constexpr uint32_t SPLIT_SMALL = (127 - 48) << 23;  // 2^-48 as bits
+__device__ __forceinline__ bool split_unsure(float v) {
+  return (__float_as_uint(v) & 0x7fffffffu) - SPLIT_SMALL >= 0x7f800000u - SPLIT_SMALL;
+}
 
-// Such elements of a weight tile's RT row tiles, taken from the fp32 instructions (wt(s), xt(s, t): the fragments of k step s);
-// the others keep their sums, so that an element depends on its own row and column alone. Called by a whole wave.
-template <int RT, class WT, class XT>
-__device__ __forceinline__ void redo_unsure(f32x4_t (&acc)[RT], int n, int N, int ksteps, WT wt, XT xt) {
+// Such elements of a wave's CT x RT tiles, taken from the fp32 instructions (wt(a, s), xt(s, t): the fragments of k step s; n: the
+// lane's first column of tile a = 0); the others keep their sums, so that an element depends on its own row and column
+// alone. Rows of zeros (raw(s, t): the row before its activation, which keeps zeros) give zeros and are no reason for it:
+// reading the rows again costs a quarter of the kernel's time (3584 x 3072 x 512 with a zero row in each tile, 83 -> 108 us, MI355X), the
+// fp32 instructions twice it (280). Called by a whole wave.
+template <int CT, int RT, class WT, class XT, class RAW>
+__device__ __forceinline__ void redo_unsure(f32x4_t (&acc)[CT][RT], int n, int N, int ksteps, WT wt, XT xt, RAW raw) {
   bool unsure = false;
 #pragma unroll
-  for (int t = 0; t < RT; ++t)
+  for (int a = 0; a < CT; ++a)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) unsure |= n + r < N && split_unsure(acc[t][r]);
+    for (int t = 0; t < RT; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) unsure |= n + 16 * a + r < N && split_unsure(acc[a][t][r]);
   if (!__ballot(unsure)) return;
-  f32x4_t f[RT];
+  uint32_t nz[RT];
 #pragma unroll
-  for (int t = 0; t < RT; ++t) f[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-  for (int s = 0; s < ksteps; ++s) {
-    const f32x8 w = wt(s);
+  for (int t = 0; t < RT; ++t) nz[t] = 0;
+#pragma unroll 2
+  for (int s = 0; s < ksteps; ++s)
 #pragma unroll
-    for (int t = 0; t < RT; ++t) f[t] = mfma16x16x32_f32(w, xt(s, t), f[t]);
+    for (int t = 0; t < RT; ++t) {
+      const f32x8 x = raw(s, t);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) nz[t] |= __float_as_uint(x.v[e]) & 0x7fffffffu;
+    }
+#pragma unroll
+  for (int t = 0; t < RT; ++t) {  // the row's four lanes
+    nz[t] |= __shfl_xor(nz[t], 16, 64);
+    nz[t] |= __shfl_xor(nz[t], 32, 64);
   }
 #pragma unroll
-  for (int t = 0; t < RT; ++t)
+  for (int a = 0; a < CT; ++a) {
+    unsure = false;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) acc[t][r] = split_unsure(acc[t][r]) ? f[t][r] : acc[t][r];
+    for (int t = 0; t < RT; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) unsure |= n + 16 * a + r < N && nz[t] && split_unsure(acc[a][t][r]);
+    if (!__ballot(unsure)) continue;
+    f32x4_t f[RT];
+#pragma unroll
+    for (int t = 0; t < RT; ++t) f[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int s = 0; s < ksteps; ++s) {
+      const f32x8 w = wt(a, s);
+#pragma unroll
+      for (int t = 0; t < RT; ++t) f[t] = mfma16x16x32_f32(w, xt(s, t), f[t]);
+    }
+#pragma unroll
+    for (int t = 0; t < RT; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[a][t][r] = split_unsure(acc[a][t][r]) ? f[t][r] : acc[a][t][r];
+  }
 }
 
 template <int WR, int RT, int CT, int EPI>  // EPI 0: plain, 1: GELU, 2: the conv epilogue
@@ -168,16 +204,15 @@ __global__ __launch_bounds__(256) void linear_f32x3_kernel(const float* __restri
     }
   }
 
-#pragma unroll
-  for (int a = 0; a < CT; ++a) {
-    const int tile = t0 + wc * CT + a;
-    redo_unsure<RT>(
-        acc[a], 16 * tile + 4 * lg, N, ksteps,
-        [&](int s) { return ldv<M3X_F32>(Wp + ((long)min(tile, ntiles - 1) * ksteps + s) * 512 + lane * 8); },
-        [&](int s, int t) {
-          return ldv<M3X_F32>(X + (long)min(m0 + 16 * (wr * RT + t) + li, M - 1) * ldx + s * 32 + 8 * lg);
-        });
-  }
+  auto xt = [&](int s, int t) {
+    return ldv<M3X_F32>(X + (long)min(m0 + 16 * (wr * RT + t) + li, M - 1) * ldx + s * 32 + 8 * lg);
+  };
+  redo_unsure<CT, RT>(
+      acc, 16 * (t0 + wc * CT) + 4 * lg, N, ksteps,
+      [&](int a, int s) {
+        return ldv<M3X_F32>(Wp + ((long)min(t0 + wc * CT + a, ntiles - 1) * ksteps + s) * 512 + lane * 8);
+      },
+      xt, xt);
 
   const bool vec = (ldy & 3) == 0 && (((uintptr_t)Y) & 15) == 0;
 #pragma unroll

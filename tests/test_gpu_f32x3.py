@@ -162,3 +162,43 @@ def test_nonfinite_rows_leave_the_others_alone(gpu):
     clean = torch.ones(B, T, dtype=torch.bool)
     clean[5, 40:43] = clean[17, :3] = clean[23, :2] = False  # a row's three taps
     assert torch.equal(a[clean], b[clean]) and not bool(b[~clean].isfinite().all(1).any())
+
+
+@pytest.mark.parametrize("e", [-60, -100, -112, -120, -126, -135])
+@pytest.mark.parametrize("which", ["x", "w"])
+def test_tiny_operands(gpu, which, e):
+    """Operands whose third (below 2^-110) or second bf16 value would be lost keep float32's accuracy: K / 4 additions and as
+    many steps of the smallest number, which is 2^-149."""
+    from m3x import ops
+    M, N, K = 1030, 1024, 64
+    g = _g(8)
+    x, w = torch.randn(M, K, generator=g), torch.randn(N, K, generator=g)
+    T, C, CN, cx, state, cw = _conv_case(160, 9)
+    if which == "x":
+        x, cx, state = (t * 2.0 ** e for t in (x, cx, state))
+    else:
+        w, cw = w * 2.0 ** e, cw * 2.0 ** e
+    def bound(s, k):
+        return (k / 4 + 4) * (2.0 ** -24 * s + 2.0 ** -149)
+    y = ops.linear(x.to(gpu), ops.pack_weight(w.to(gpu))).cpu().double()
+    ref, s = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    assert bool(((y - ref).abs() <= bound(s, K)).all())
+    slots = torch.arange(160, device=gpu)
+    y = ops.conv_gemm(cx.to(gpu), ops.pack_weight(cw.to(gpu)), torch.empty(160 * T, CN, device=gpu),
+                      gather=(state.to(gpu), slots, T, C, 1, False)).cpu().double()
+    j = torch.cat([state.double().view(160, 2, C), cx.double().view(160, T, C)], 1)
+    cols = torch.cat([j[:, i:i + T] for i in range(3)], 2).view(160 * T, 3 * C)
+    ref, s = cols @ cw.double().t(), cols.abs() @ cw.double().abs().t()
+    assert bool(((y - ref).abs() <= bound(s, 3 * C)).all())
+
+
+def test_zero_rows_and_odd_columns(gpu):
+    """Rows of zeros give zeros (signs and all finite), beside others, at a column count that is no multiple of 16."""
+    from m3x import ops
+    M, N, K = 2500, 515, 96
+    g = _g(10)
+    x, w = torch.randn(M, K, generator=g), torch.randn(N, K, generator=g)
+    x[100:300] = 0
+    y = ops.linear(x.to(gpu), ops.pack_weight(w.to(gpu))).cpu().double()
+    ref, s = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    assert not bool(y[100:300].any()) and bool(((y - ref).abs() <= _bound(s, K)).all())
