@@ -980,7 +980,11 @@ __global__ __launch_bounds__(256) void linear_strip_kernel(const uint16_t* __res
   // The epilogue's row operands are read here, with the first stages' loads, and kept in LDS, so that no global
   // round trip is left after the products: EPI_QKR's positions and slots (loads clamped to valid rows, no branch
   // around them) and PRO's row scale and shift (measured at 2264 rows inside the mixed step: gate|up + SwiGLU +
-  // norm 45.9 -> 43.0 us, q|k|v + norm + RoPE + cache 38.5 -> 33.0 us).
+  // norm 45.9 -> 43.0 us, q|k|v + norm + RoPE + cache 38.5 -> 33.0 us). The narrow plain tiles take the scale and shift
+  // behind stage 0's products instead of making the first stage wait for the statistics (416 x 3072 x 1024, 32 x 64 tiles
+  // 11.1 -> 9.1 us, 64 x 64 11.8 -> 10.4; the chunked plan 9.9); in the others the statistics' registers, held that long,
+  // cost a workgroup per CU.
+  constexpr bool LATE = PRO && !DUAL && NG == 1;
   int qps = 0;
   long qsl = 0;
   if constexpr (EPI == EPI_QKR) {
@@ -1001,19 +1005,22 @@ __global__ __launch_bounds__(256) void linear_strip_kernel(const uint16_t* __res
       ssl[tid] = qsl;
     }
   }
-  if constexpr (PRO) ns.finish(ni, m0, M, PRO_K, pst);
+  if constexpr (PRO && !LATE) ns.finish(ni, m0, M, PRO_K, pst);
   astore(la0, A0);
   __syncthreads();
   // Stage s issues the weights (register set s + 2 mod 3) and activations (set s mod 2, stored to LDS during stage
   // s - 1) of stage s + 2, multiplies stage s (weights from set s mod 3, activations from LDS buffer s mod 2),
   // stores stage s + 1's activations to the other buffer, then meets the workgroup: unrolled by 6.
-#define M3X_STRIP_STAGE(S, WN, WC, AN, AS, BUF, OBUF) \
-  if (s0 + S < nst) {                                 \
-    wload(s0 + S + 2, WN);                            \
-    aload(s0 + S + 2, AN);                            \
-    compute(BUF, WC);                                 \
-    if (s0 + S + 1 < nst) astore(OBUF, AS);           \
-    __syncthreads();                                  \
+#define M3X_STRIP_STAGE(S, WN, WC, AN, AS, BUF, OBUF)          \
+  if (s0 + S < nst) {                                          \
+    wload(s0 + S + 2, WN);                                     \
+    aload(s0 + S + 2, AN);                                     \
+    compute(BUF, WC);                                          \
+    if constexpr (LATE && S == 0) {                            \
+      if (s0 == 0) ns.finish(ni, m0, M, PRO_K, pst);           \
+    }                                                          \
+    if (s0 + S + 1 < nst) astore(OBUF, AS);                    \
+    __syncthreads();                                           \
   }
   for (int s0 = 0; s0 < nst; s0 += 6) {
     M3X_STRIP_STAGE(0, W2, W0, A0, A1, la0, la1)
@@ -1256,9 +1263,10 @@ static bool launch_linear(const LinearPlan& p, hipStream_t st, const uint16_t* X
                           const uint16_t* W2, uint16_t* Y, long ldy, int M, int N, int K, const NormIn& ni = NormIn{},
                           const ResidOut& ro = ResidOut{}, const QkOut& qk = QkOut{}) {
   static_assert(!(PRO && EPI == EPI_RESID), "a residual projection takes its input as is");
-  // up to 512 rows a folded norm's statistics delay the strips' first stage: 416 x 3072 x 1024 inside the depth frame 16.4
-  // (plain) and 17.5 us (GELU) against 13.0 and 14.2 with the chunked plan, SwiGLU even. The bf16 q|k|v stays on the
-  // strips with its fused epilogue, and the plain product with it (same bits).
+  // Up to 512 rows the bf16 q|k|v with a folded norm takes the strips for its fused epilogue, and the plain product with it
+  // (same bits; 416 x 3072 x 1024 9.1 us, chunked 9.9). The others keep the chunked plan: SwiGLU is even (416 rows 16.3, 16.4 us),
+  // and the GELU and fp16 products were when a strip's first stage waited for the statistics (416 x 3072 x 1024 GELU 11.9
+  // us, 9.8 since, chunked 10.8).
   constexpr bool CHUNKED = PRO && !(DT == M3X_BF16 && (EPI == EPI_QKR || EPI == EPI_NONE));
   const StripTile t = CHUNKED && M <= 512 ? StripTile{0, 0} : strip_tile<EPI>(M, N, K, ldx);
   if (t.rt) {

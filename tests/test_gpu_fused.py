@@ -85,7 +85,7 @@ def _act_ref(a, u, act, dtype):
     return a
 
 
-@pytest.mark.parametrize("M", [1, 3, 16, 64, 130, 224, 600, 2264])
+@pytest.mark.parametrize("M", [1, 3, 16, 64, 130, 224, 257, 400, 512, 600, 2264])
 @pytest.mark.parametrize("act,kind", [(-1, 1), (0, 1), (1, 0), (-1, 0)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_linear_normed(gpu, M, act, kind, dtype):
