@@ -1111,21 +1111,31 @@ __global__ __launch_bounds__(256) void linear_strip_kernel(const uint16_t* __res
   }
 }
 
-// The strip kernel's tile (RT row tiles x 4 NG weight tiles) for M rows of N columns, rt = 0: another plan. The largest
-// of the tiles whose grid keeps the chip busy; graph-timed on MI355X, us (tile: time, blocks in brackets):
-//   plain    2264 x 4096 x 1024: 80 x 256 26.6 (464), 64 x 128 30.5 (1152); 1024 x 4096 x 1024: 16.8 (208), 14.2 (512);
-//            30720 x 512 x 128: 17.8 (768), 19.5 (1920); 3584 x 3072 x 512: 27.2 (540: a second round of two a CU, nearly
-//            empty), 24.6 (1344). So 80 x 256 for one full round or many.
-//            416 x 3072 x 1024 GELU: 32 x 64 10.1 (624), 64 x 64 11.5 (336); 700 x 3072 x 512: 9.4 (1056), 8.7 (528)
-//            1024 x 256 x 1536: 32 x 64 6.5 (128), 64 x 64 8.5 (64), 64 x 128 11.9 (32); 3584 x 256 x 1536: 10.4 (448),
-//            10.3 (224), 12.2 (112)
-//   SwiGLU   1500 x 3072 x 1024: 80-row pairs of strips 24.0 (456), 64 rows x 64 columns 26.8 (1152); 512 rows: 15.8, 12.4
-//   residual 2264 x 1024 x 2048: 80 x 128 21.7 (232), 64 x 64 26.0 (576); 1024 rows: 20.8, 13.2 (256), 32 x 64 13.7 (512);
-//            640 rows: 20.4, 12.0 (160), 11.0 (320)
-// (bf16 at K = 1024 and more, fp16 below.) The 8-wave 128 x 128 tiles with both operands in LDS that such shapes took
-// before were slower at every one of them but 6144 x 1280 x 256 (13.6 against 14.2). Up to 512 rows the K-split plans
-// win unless 32 x 64 blocks fill the chip: 448 x 1536 x 512 4.7 (336 blocks) against 5.2, 448 x 512 x 512 4.0 (112)
-// against 3.3, residual 512 x 1024 x 2048 10.0 (256) against 9.9.
+// The strip kernel's tile (RT row tiles x 4 NG weight tiles) for M rows of N columns, rt = 0: another plan. A grid takes as
+// many rounds of 256 workgroups (one a CU) as it starts, so the large tile is chosen where its rounds are few enough beside
+// the small one's; graph-timed on MI355X with weights not in the caches, us (tile: time, workgroups in brackets):
+//   plain    80 x 256 is about two rounds of 64 x 128, an odd one half more (a lone workgroup a CU overlaps with nothing):
+//            1120 x 4096 x 1024 16.8 (224), 18.5 (576); 1024 rows 16.4 (208), 14.8 (512); 2016 rows 25.2 (416), 27.0 (1024);
+//            1500 rows 23.9 (304), 20.7 (768); 3584 rows 39.9 (720), 44.4 (1792); 2688 rows 37.9 (544), 36.2 (1344);
+//            2264 x 2048 x 1024 17.3 (232), 20.0 (576). Only the lines at 440 and 740 workgroups before: 8 to 16 % slower
+//            than the 80-row blocks alone at 1120, 2016, 3136 and 3584 rows.
+//            700 x 3072 x 512: 32 x 64 9.4 (1056), 64 x 64 8.7 (528); 1024 x 256 x 1536: 6.5 (128), 8.5 (64), 64 x 128 11.9 (32);
+//            3584 x 256 x 1536: 10.4 (448), 10.3 (224), 12.2 (112)
+//   q|k|v    with its epilogue (4096 columns, K = 1024, folded norm): never 80 x 256 in one round (1120 rows 23.1, 20.9); 1792 rows 30.6
+//            (368), 29.2 (896); 2016 rows 31.3 (416), 33.6 (1024); 2688 rows 48.0 (544), 42.0 (1344); 3584 rows 50.8 (720), 56.0 (1792)
+//   GELU     the epilogue (erff) of a large tile is long and the last one stands alone: 80 x 256 only for a full even round:
+//            3136 x 3072 x 1024 36.4 (480), 64 x 128 38.3 (1176); 2264 rows 32.9 (348), 31.4 (864); 6944 rows 87.6 (1044), 81.2 (2616).
+//            64 x 128 against 64 x 64: 1120 rows 17.0 (432), 17.7 (864); 896 rows 16.1 (336), 15.5 (672); at K = 512 the products are
+//            too short to hide it: 3136 x 2048 x 512 22.8 (784), 18.7 (1568); 6944 rows 39.4 (1744), 41.6 (3488)
+//   SwiGLU   80-row pairs of strips (80 x 128) against 64 x 64 (3072 columns, K = 1024): 800 rows 18.2 (240), 19.3 (624); 600 rows 17.8
+//            (192), 14.3 (480); 896 rows 22.2 (288), 19.6 (672); 1120 rows 22.6 (336), 24.7 (864); 2016 rows 36.2 (624), 37.5 (1536);
+//            1500 x 2816 x 1024 27.3 (418), 32.2 (1056) with the norm
+//   residual 2264 x 1024 x 1024: 80 x 128 14.9 (232), 64 x 64 17.0 (576); 2016 rows 14.6 (208), 12.7 (512); 2688 rows 21.2 (272), 17.6
+//            (672); 3136 rows 21.7 (320), 21.9 (784); 640 x 1024 x 2048: 20.4, 12.0 (160), 32 x 64 11.0 (320)
+// Up to 512 rows the K-split plans win unless 32 x 64 blocks fill the chip: 448 x 1536 x 512 4.7 (336 blocks) against 5.2,
+// 448 x 512 x 512 4.0 (112) against 3.3; GELU 320 x 2048 x 512 5.9 (320) against 5.3, 416 rows 6.0 (416) against 6.2.
+// The 8-wave 128 x 128 tiles with both operands in LDS that fp16 took before are faster in a few spots: 2264 x 3072 x 1024 GELU 28.7
+// against 31.4, 2688 x 3072 x 1024 28.2 against 29.8.
 struct StripTile {
   int rt, ng;
 };
@@ -1134,22 +1144,27 @@ static StripTile strip_tile(int M, int N, int K, long ldx) {
   // 32-bit element offsets into the packed weight and the activations; whole K stages
   if (M <= 256 || K % 64 || (long)m3x_ceil_div(N, 16) * 16 * K >= (1L << 31) || (long)M * ldx >= (1L << 31)) return {0, 0};
   auto blocks = [&](int rt, int ng) { return (long)m3x_ceil_div(M, 16 * rt) * m3x_ceil_div(N, 64 * ng); };
-  if (M <= 512 && blocks(2, 1) < 300) return {0, 0};
+  auto rounds = [&](int rt, int ng) { return (blocks(rt, ng) + 255) / 256; };
+  if (M <= 512 && blocks(2, 1) < (EPI == EPI_GELU ? 380 : 300)) return {0, 0};
   if constexpr (EPI == EPI_QKR) {
-    const long b = blocks(5, 4);
-    if (N % 256 == 0 && ((b >= 440 && b <= 512) || b >= 740)) return {5, 4};
+    const long r = rounds(5, 4);
+    if (N % 256 == 0 && r >= 2 && blocks(4, 2) >= 480 * r) return {5, 4};
     return N % 128 == 0 ? StripTile{4, 2} : StripTile{0, 0};
-  } else if constexpr (EPI == EPI_SWIGLU) {
-    if (blocks(5, 2) >= 440) return {5, 2};
-  } else if constexpr (EPI == EPI_RESID) {
-    if (blocks(4, 1) > 480) return {5, 2};
+  } else if constexpr (EPI == EPI_SWIGLU || EPI == EPI_RESID) {
+    const long r = rounds(5, 2);
+    if (rounds(4, 1) >= 2 * r + (r == 1)) return {5, 2};
+    return blocks(4, 1) >= 200 ? StripTile{4, 1} : StripTile{2, 1};
   } else {
-    const long b = blocks(5, 4);
-    if ((b >= 440 && b <= 512) || b >= 740) return {5, 4};
-    if (blocks(4, 2) >= 250) return {4, 2};
+    const long r = rounds(5, 4), r42 = rounds(4, 2);
+    if constexpr (EPI == EPI_GELU) {
+      if (K >= 1024 && r % 2 == 0 && r42 > 2 * r) return {5, 4};
+      if (blocks(4, 2) >= (K >= 1024 ? 400 : 1600)) return {4, 2};
+    } else {
+      if (r42 >= 2 * r + r % 2) return {5, 4};
+      if (blocks(4, 2) >= 250) return {4, 2};
+    }
     return blocks(4, 1) >= 400 ? StripTile{4, 1} : StripTile{2, 1};
   }
-  return blocks(4, 1) >= 200 ? StripTile{4, 1} : StripTile{2, 1};
 }
 
 struct LinearPlan {
