@@ -1197,8 +1197,10 @@ static bool wide_plan(int M, int N, int K, bool dual, LinearPlan& p) {
     return true;
   }
   const int ntiles = m3x_ceil_div(N, 16);
-  if (M > 256 && M <= 512 && K == 2048 && !dual && (long)m3x_ceil_div(M, 32) * m3x_ceil_div(ntiles, 4) <= 256) {
-    // 32-row blocks of 16 waves in one round (512 x 1024 x 2048 with the residual: 8.5 against 9.9 us chunked)
+  const long wgs32 = (long)m3x_ceil_div(M, 32) * m3x_ceil_div(ntiles, 4);
+  if (M > 256 && M <= 512 && K == 2048 && !dual && wgs32 > 128 && wgs32 <= 256) {
+    // 32-row blocks of 16 waves in one round that fills half the chip (512 x 1024 x 2048 with the residual: 8.5 against 9.9
+    // us chunked; 300 x 512 x 2048, 80 workgroups, 7.1 against 6.4)
     p.mt = 2;
     p.nw = 4;
     p.nwaves = 16;
