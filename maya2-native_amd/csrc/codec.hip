@@ -440,22 +440,19 @@ __global__ __launch_bounds__(256) void conv_x3_kernel(const float* __restrict__ 
     }
   }
   if (wave > lastw) return;  // rows past T, never stored (no barrier follows)
-  auto row = [&](int s, int t) { return t0 + min(16 * (wave * RT + t) + li + s / cst * cs.dil, rows - 1); };
-  auto raw = [&](int s, int t) {
-    const int i = row(s, t), c = 32 * (s % cst) + 8 * lg;
-    return ldv<M3X_F32>(i < cs.pad ? hs + (long)i * cs.C + c : xs + (long)i * ldx + c);
-  };
   redo_unsure<CT, RT>(
-      acc, n0, n0 + 16 * CT, ks, [&](int a, int s) { return ldv<M3X_F32>(wb + ((long)a * ks + s) * 512); },
+      acc, ks, [&](int a, int s) { return ldv<M3X_F32>(wb + ((long)a * ks + s) * 512); },
       [&](int s, int t) {
-        f32x8 x = raw(s, t);
-        if (cs.pre_elu && row(s, t) >= cs.pad) {
+        const int tap = s / cst;
+        const int i = t0 + min(16 * (wave * RT + t) + li + tap * cs.dil, rows - 1);
+        const int c = 32 * (s - tap * cst) + 8 * lg;
+        f32x8 x = ldv<M3X_F32>(i < cs.pad ? hs + (long)i * cs.C + c : xs + (long)i * ldx + c);
+        if (cs.pre_elu && i >= cs.pad) {
 #pragma unroll
           for (int e = 0; e < 8; ++e) x.v[e] = elu<M3X_F32>(x.v[e]);
         }
         return x;
-      },
-      raw);
+      });
 #pragma unroll
   for (int t = 0; t < RT; ++t) {
     const int tr = t0 + 16 * (wave * RT + t) + li;

@@ -45,7 +45,10 @@ struct F32Epi {
 // Results that the split cannot give as fp32 would are taken from the fp32 instructions, element by element (redo_unsure):
 // those that are not finite (an infinity or NaN in the operands, or a value that bf16(x) rounds to infinity), and those
 // below 2^-48, where what the split loses of operands below 2^-110 (up to 2^-134 times the other operand's sum) may be more
-// than fp32's rounding. Before, x of 2^-126 N(0, 1) came out 2e-3 off and x of 2^-136 N(0, 1) as zeros, 2.9e-7 and 3.5e-5 in fp32.
+// than fp32's rounding: x of 2^-126 N(0, 1) came out 2e-3 off, 2.9e-7 in fp32. A sum of exactly zero stands: it is a row of
+// zeros or a cancellation (one in 10^7 to 10^8 sums, each of which would hold its launch up by a redone tile: 12.7 -> 16.3 us
+// at 19200 x 64 x 256); if its operands are below 2^-110 all the same, it is off by up to the 2^-134 above, and operands
+// below 2^-134, deep in fp32's subnormals, count as zero.
 __device__ __forceinline__ void split_bf16x3(const f32x8& x, u16x8& h, u16x8& m, u16x8& l) {
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
@@ -68,50 +71,33 @@ __device__ __forceinline__ void mfma_x3(const u16x8 (&w)[3], const u16x8 (&b)[RT
     for (int t = 0; t < RT; ++t) acc[t] = mfma16x16x32<M3X_BF16>(w[PW[i]], b[t][PX[i]], acc[t]);
 }
 
-// Whether a split sum may be worse than fp32's: it is not finite, or below 2^-48 (zero included).
+// Whether a split sum may be worse than fp32's: it is not finite, or below 2^-48 and not zero.
 constexpr uint32_t SPLIT_SMALL = (127 - 48) << 23;  // 2^-48 as bits
 __device__ __forceinline__ bool split_unsure(float v) {
-  return (__float_as_uint(v) & 0x7fffffffu) - SPLIT_SMALL >= 0x7f800000u - SPLIT_SMALL;
+  const uint32_t a = __float_as_uint(v) & 0x7fffffffu;
+  return a - SPLIT_SMALL >= 0x7f800000u - SPLIT_SMALL && a != 0;
 }
 
-// Such elements of a wave's CT x RT tiles, taken from the fp32 instructions (wt(a, s), xt(s, t): the fragments of k step s; n: the
-// lane's first column of tile a = 0); the others keep their sums, so that an element depends on its own row and column
-// alone. Rows of zeros (raw(s, t): the row before its activation, which keeps zeros) give zeros and are no reason for it:
-// reading the rows again costs a quarter of the kernel's time (3584 x 3072 x 512 with a zero row in each tile, 83 -> 108 us, MI355X), the
-// fp32 instructions twice it (280). Called by a whole wave.
-template <int CT, int RT, class WT, class XT, class RAW>
-__device__ __forceinline__ void redo_unsure(f32x4_t (&acc)[CT][RT], int n, int N, int ksteps, WT wt, XT xt, RAW raw) {
-  bool unsure = false;
+// Such elements of a wave's CT x RT tiles, taken from the fp32 instructions (wt(a, s), xt(s, t): the fragments of k step s); the
+// others keep their sums, so that an element depends on its own row and column alone. Called by a whole wave.
+template <int CT, int RT, class WT, class XT>
+__device__ __forceinline__ void redo_unsure(f32x4_t (&acc)[CT][RT], int ksteps, WT wt, XT xt) {
+  // most tiles hold none, nor zeros: 1.5 operations an element (the magnitude from SPLIT_SMALL on, doubled)
+  uint32_t far = 0;
 #pragma unroll
   for (int a = 0; a < CT; ++a)
 #pragma unroll
     for (int t = 0; t < RT; ++t)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) unsure |= n + 16 * a + r < N && split_unsure(acc[a][t][r]);
-  if (!__ballot(unsure)) return;
-  uint32_t nz[RT];
-#pragma unroll
-  for (int t = 0; t < RT; ++t) nz[t] = 0;
-#pragma unroll 2
-  for (int s = 0; s < ksteps; ++s)
-#pragma unroll
-    for (int t = 0; t < RT; ++t) {
-      const f32x8 x = raw(s, t);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) nz[t] |= __float_as_uint(x.v[e]) & 0x7fffffffu;
-    }
-#pragma unroll
-  for (int t = 0; t < RT; ++t) {  // the row's four lanes
-    nz[t] |= __shfl_xor(nz[t], 16, 64);
-    nz[t] |= __shfl_xor(nz[t], 32, 64);
-  }
+      for (int r = 0; r < 4; ++r) far = max(far, (__float_as_uint(acc[a][t][r]) << 1) - (SPLIT_SMALL << 1));
+  if (!__ballot(far >= (0x7f800000u - SPLIT_SMALL) << 1)) return;
 #pragma unroll
   for (int a = 0; a < CT; ++a) {
-    unsure = false;
+    bool unsure = false;
 #pragma unroll
     for (int t = 0; t < RT; ++t)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) unsure |= n + 16 * a + r < N && nz[t] && split_unsure(acc[a][t][r]);
+      for (int r = 0; r < 4; ++r) unsure |= split_unsure(acc[a][t][r]);
     if (!__ballot(unsure)) continue;
     f32x4_t f[RT];
 #pragma unroll
@@ -204,15 +190,14 @@ __global__ __launch_bounds__(256) void linear_f32x3_kernel(const float* __restri
     }
   }
 
-  auto xt = [&](int s, int t) {
-    return ldv<M3X_F32>(X + (long)min(m0 + 16 * (wr * RT + t) + li, M - 1) * ldx + s * 32 + 8 * lg);
-  };
   redo_unsure<CT, RT>(
-      acc, 16 * (t0 + wc * CT) + 4 * lg, N, ksteps,
+      acc, ksteps,
       [&](int a, int s) {
         return ldv<M3X_F32>(Wp + ((long)min(t0 + wc * CT + a, ntiles - 1) * ksteps + s) * 512 + lane * 8);
       },
-      xt, xt);
+      [&](int s, int t) {
+        return ldv<M3X_F32>(X + (long)min(m0 + 16 * (wr * RT + t) + li, M - 1) * ldx + s * 32 + 8 * lg);
+      });
 
   const bool vec = (ldy & 3) == 0 && (((uintptr_t)Y) & 15) == 0;
 #pragma unroll

@@ -107,7 +107,7 @@ def test_conv_gemm_f32_gathered(gpu, B, T, C, N, dil, pre):
 
 
 @pytest.mark.parametrize("M,N,K", [(10240, 64, 32), (10303, 64, 96), (5130, 128, 64), (16000, 128, 32), (16321, 64, 96),
-                                   (16320, 64, 96), (8130, 128, 64)])
+                                   (16320, 64, 96), (16321, 128, 64), (16320, 128, 64)])
 def test_conv_gemm_f32_plain(gpu, M, N, K):
     from m3x import ops
     g = _g(M + N + K)
@@ -164,7 +164,7 @@ def test_nonfinite_rows_leave_the_others_alone(gpu):
     assert torch.equal(a[clean], b[clean]) and not bool(b[~clean].isfinite().all(1).any())
 
 
-@pytest.mark.parametrize("e", [-60, -100, -112, -120, -126, -135])
+@pytest.mark.parametrize("e", [-60, -100, -112, -120, -126])
 @pytest.mark.parametrize("which", ["x", "w"])
 def test_tiny_operands(gpu, which, e):
     """Operands whose third (below 2^-110) or second bf16 value would be lost keep float32's accuracy: K / 4 additions and as
