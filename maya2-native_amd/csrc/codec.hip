@@ -1097,9 +1097,10 @@ M3X_API int m3x_conv_gemm(const void* x, long ldx, const void* w_packed, const v
       M3X_CHECK_LAUNCH();
       return M3X_OK;
     }
-    // plain rows (a 1x1 conv, or gathered columns): the projection's kernel with the conv epilogue
+    // plain rows (a 1x1 conv, or gathered columns): the projection's kernel with the conv epilogue, from a workgroup a CU:
+    // 15360 x 128 x 64 (240) 12.0 against 10.8 us, 19200 (300) 13.4 against 15.0 (in place)
     const int mblk = m3x_ceil_div(M, 64), nblk = N / 64;
-    if (!G && N >= 64 && y != x && (long)mblk * nblk >= F32X3_MIN_BLOCKS) {
+    if (!G && N >= 64 && y != x && mblk >= F32X3_MIN_BLOCKS) {
       if (N == 128)
         hipLaunchKernelGGL((linear_f32x3_kernel<2, 2, 4, 2>), dim3((unsigned)xcd_grid(mblk, 1)), dim3(256), 0, st, X, ldx,
                            W, (float*)y, ldy, M, N, K, mblk, 1, ep);
