@@ -144,14 +144,16 @@ __device__ float radix_kth(const float (&x)[NE], int V, int k, SM& sm) {
 }
 
 // The k-th largest of 256 values held 4 a lane by every wave, approximately: a value t with at least k of them >= t,
-// at most k + k / 16 unless values repeat or crowd within the search's reach. lo: a value with count(>= lo) >= k.
-// Three thresholds a round (their counts are independent, a round is bound by the latency of one): 4-5 rounds.
+// at most max(k + k / 16, 40) unless values repeat or crowd within the search's reach. lo: a value with count(>= lo) >= k.
+// Three thresholds a round (their counts are independent, a round is bound by the latency of one): up to 4-5 rounds. It
+// ends where the interval is a step of a bf16 value: repeats at the k-th place would keep it going to no purpose (224 flat
+// rows of 2048, k = 10: 6.8 us with the search run to its end, 5.2 so).
 __device__ __forceinline__ float wave_kth(const float (&c)[4], float lo, float hi, int k) {
-  const int enough = k + (k >> 4);
+  const int enough = max(k + (k >> 4), 40);
   for (int it = 0; it < 12; ++it) {
     const float m2 = 0.5f * lo + 0.5f * hi;
     const float m1 = 0.5f * lo + 0.5f * m2, m3 = 0.5f * m2 + 0.5f * hi;
-    if (!(m2 > lo && m2 < hi)) break;
+    if (!(m2 > lo && m2 < hi && hi - lo > 0x1p-8f * fabsf(m2))) break;
     int n1 = 0, n2 = 0, n3 = 0;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -240,10 +242,11 @@ __device__ bool hist_marks(const float (&x)[NE], int V, int k, float m, SM& sm, 
 // k = 50 of 2048. It needs no atomics and one barrier, whatever the shape of the row; a histogram of the distances below
 // the maximum serialised its atomics on a peaked row, whose bulk falls into a few bins. Rows of 2048 with one code 16
 // above the bulk, MI355X: the 224-seat depth frame (30 such samplers) 5.11 -> 4.94 ms, the one-seat frame 2.35 ->
-// 2.21 ms; head and codebook-0 sampler of 224 flat rows 24.2 -> 21.4 and 24.5 -> 22.8 us in two runs (repeats of one
-// build differ by 7 to 14 % there). Larger k takes the histogram: the maxima would let through several times k candidates
-// (k = 200 of 2048: about 350). More than 256 candidates (an order that gathers the leaders in a few threads, many
-// repeats), or fewer than k threads with a maximum above -inf, take the exact radix select.
+// 2.21 ms. The sampler alone, us, 224 rows, histogram / maxima: peaked k = 10 6.8 / 5.2, 50 8.9 / 6.0, 100 11.6 / 10.2; flat k = 10
+// 5.8 / 5.2, 50 5.9 / 5.8, 80 8.8 / 6.7, 100 9.3 / 10.2, 128 10.8 / 12.3 (more than 128 candidates, ranked one a thread). Larger k
+// takes the histogram: the maxima would let through several times k candidates (k = 200 of 2048: about 350). More than 256
+// candidates (an order that gathers the leaders in a few threads, many repeats), or fewer than k threads with a maximum
+// above -inf, take the exact radix select.
 // The kernel runs every line of code once or twice a launch, so it is bound by latencies (dependent operations, barriers,
 // instruction fetch) and short loops beat unrolled code.
 constexpr int KFAST = 128;
