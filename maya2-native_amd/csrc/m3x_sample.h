@@ -145,15 +145,16 @@ __device__ float radix_kth(const float (&x)[NE], int V, int k, SM& sm) {
 
 // The k-th largest of 256 values held 4 a lane by every wave, approximately: a value t with at least k of them >= t,
 // at most max(k + k / 16, 40) unless values repeat or crowd within the search's reach. lo: a value with count(>= lo) >= k.
-// Three thresholds a round (their counts are independent, a round is bound by the latency of one): up to 4-5 rounds. It
-// ends where the interval is a step of a bf16 value: repeats at the k-th place would keep it going to no purpose (224 flat
-// rows of 2048, k = 10: 6.8 us with the search run to its end, 5.2 so).
+// Three thresholds a round (their counts are independent, a round is bound by the latency of one): up to 4-5 rounds. Six
+// narrow a row's range to its 4096th part, a step of a bf16 value or less; with repeats at the k-th place more come to
+// nothing (224 flat rows of 2048, k = 10: 6.9 us with twelve rounds, 5.1 so). Unrolled, the one-seat depth frame loses 0.4 %.
 __device__ __forceinline__ float wave_kth(const float (&c)[4], float lo, float hi, int k) {
   const int enough = max(k + (k >> 4), 40);
-  for (int it = 0; it < 12; ++it) {
+#pragma unroll 1
+  for (int it = 0; it < 6; ++it) {
     const float m2 = 0.5f * lo + 0.5f * hi;
     const float m1 = 0.5f * lo + 0.5f * m2, m3 = 0.5f * m2 + 0.5f * hi;
-    if (!(m2 > lo && m2 < hi && hi - lo > 0x1p-8f * fabsf(m2))) break;
+    if (!(m2 > lo && m2 < hi)) break;
     int n1 = 0, n2 = 0, n3 = 0;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -242,8 +243,8 @@ __device__ bool hist_marks(const float (&x)[NE], int V, int k, float m, SM& sm, 
 // k = 50 of 2048. It needs no atomics and one barrier, whatever the shape of the row; a histogram of the distances below
 // the maximum serialised its atomics on a peaked row, whose bulk falls into a few bins. Rows of 2048 with one code 16
 // above the bulk, MI355X: the 224-seat depth frame (30 such samplers) 5.11 -> 4.94 ms, the one-seat frame 2.35 ->
-// 2.21 ms. The sampler alone, us, 224 rows, histogram / maxima: peaked k = 10 6.8 / 5.2, 50 8.9 / 6.0, 100 11.6 / 10.2; flat k = 10
-// 5.8 / 5.2, 50 5.9 / 5.8, 80 8.8 / 6.7, 100 9.3 / 10.2, 128 10.8 / 12.3 (more than 128 candidates, ranked one a thread). Larger k
+// 2.21 ms. The sampler alone, us, 224 rows, histogram / maxima: peaked k = 10 6.8 / 5.1, 50 8.9 / 5.7, 100 11.6 / 10.0; flat k = 10
+// 5.8 / 5.1, 50 6.0 / 5.6, 80 8.8 / 6.6, 100 9.3 / 10.1, 128 10.8 / 12.1 (more than 128 candidates, ranked one a thread). Larger k
 // takes the histogram: the maxima would let through several times k candidates (k = 200 of 2048: about 350). More than 256
 // candidates (an order that gathers the leaders in a few threads, many repeats), or fewer than k threads with a maximum
 // above -inf, take the exact radix select.
