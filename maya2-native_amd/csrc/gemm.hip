@@ -205,9 +205,10 @@ __global__ __launch_bounds__(256) void linear_f32_kernel(const float* __restrict
 // fp32 projections of up to 16 rows (a few Mimi seats): one workgroup of 16 waves per weight tile, a sixteenth of K each.
 // A wave loads its S weight fragments and the matching activations (straight into the B operand; rows past M repeat
 // row M - 1) at once, so the kernel pays one memory round trip however long K is (S = 8, K above 2048, is over its 128
-// registers: 4 of them go through scratch memory); the 16 partial tiles meet in LDS and are added in slice order. Against 4 waves walking chunks of 4 steps (MI355X, weights not in L2, us): 2 x 512 x 512 3.5 ->
-// 2.8, 2 x 512 x 2048 7.6 -> 5.6, 2 x 1024 x 3584 13.3 -> 9.9, 2 x 8192 x 1024 13.0 -> 7.8, 16 x 512 x 2048 8.2 -> 7.2. Bound by
-// the launch and by what one CU streams from behind its L2 (~25 GB/s: 128 KB a workgroup at K = 2048).
+// registers: 4 of them go through scratch memory); the 16 partial tiles meet in LDS and are added in slice order. Against
+// 4 waves walking chunks of 4 steps (MI355X, weights not in L2, us): 2 x 512 x 512 3.5 -> 2.8, 2 x 512 x 2048 7.6 -> 5.6,
+// 2 x 1024 x 3584 13.3 -> 9.9, 2 x 8192 x 1024 13.0 -> 7.8, 16 x 512 x 2048 8.2 -> 7.2. Bound by the launch and by what one CU
+// streams from behind its L2 (~25 GB/s: 128 KB a workgroup at K = 2048).
 template <int S, int EPI>
 __global__ __launch_bounds__(1024) void linear_f32_rows_kernel(const float* __restrict__ X, long ldx,
                                                                const float* __restrict__ Wp, float* __restrict__ Y,

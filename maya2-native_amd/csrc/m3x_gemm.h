@@ -1068,7 +1068,7 @@ __global__ __launch_bounds__(256) void linear_strip_kernel(const uint16_t* __res
       for (int j = 0; j < RT; ++j) {
         qk_stage(tile, LDT, 16 * j + li, 16 * (wave * NG + i) + 4 * lg, acc[0][i][j]);
         const int m = m0 + 16 * j + li;
-        if (Y && m < M)  // the projection itself, for callers that read it (uniform)
+        if (Y && m < M)  // the projection itself, where m3x_linear_qk_rope says that qkv holds it (uniform)
           qk_stage(Y + (long)m * ldy, 0, 0, (t0 + i) * 16 + 4 * lg, acc[0][i][j]);
       }
     __syncthreads();

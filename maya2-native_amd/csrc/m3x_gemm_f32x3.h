@@ -32,8 +32,8 @@ struct F32Epi {
 // 2.3e-7 at K = 256 and 9.3e-7 at K = 3584, where the fp32 instructions give 2.9e-7 and 1.07e-6 (MI355X; about the
 // same for ELU outputs, lower for rows with an offset).
 //
-// A workgroup of 4 waves (WR along the rows, 4 / WR along the columns) owns 16 RT WR rows, a wave 16 RT x 16 CT. Per k step every thread splits
-// its share of both operands once and stores the three planes to LDS as fragments (a lane's 16 bytes in lane order; the
+// A workgroup of 4 waves (WR along the rows, 4 / WR along the columns) owns 16 RT WR rows, a wave 16 RT x 16 CT. Per k step
+// every thread splits its share of both operands once and stores the three planes to LDS as fragments (a lane's 16 bytes in lane order; the
 // activations' slots XOR-swizzled so that 4 threads of a row and 4 rows hit 16 bank groups), so the split's VALU work
 // is shared by the four waves and each fragment read is one contiguous 1 KB. The next step's global loads are in
 // flight while the current one multiplies; one small LDS buffer, so that several workgroups a CU overlap one's staging

@@ -124,8 +124,8 @@ def linear_qk_rope(x, w, qkv, q_out, k_cache, v_cache, slots, pos, cos, sin, wq,
                    part=None, eps_in=0.0):
     """The q|k|v projection (x @ W.T, or with part given linear_normed's RMSNorm-folded product, W from fold_norm)
     followed by qk_norm_rope_cache on its output, in one launch when the row count's plan holds whole heads per
-    workgroup (then qkv is not written), else two through qkv. Same bits as linear / linear_normed +
-    qk_norm_rope_cache."""
+    workgroup (above 192 rows at N = 4096), else two through qkv. qkv holds the projection afterwards at up to 192 and at
+    257..512 rows. Same bits as linear / linear_normed + qk_norm_rope_cache."""
     M, K, qkv = _lin_args(x, w, qkv, w.N)
     _dev(q_out, k_cache, v_cache, slots, pos, cos, sin, wq, wk, part)
     _index(slots=slots, pos=pos)
