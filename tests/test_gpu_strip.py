@@ -10,7 +10,8 @@ import torch.nn.functional as F
 pytestmark = pytest.mark.gpu
 EPS = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}
 SHAPES = [(257, 4096, 1024), (300, 1040, 64), (511, 3072, 1024), (512, 2816, 128), (513, 1000, 192), (640, 1024, 2048),
-          (1030, 256, 1536), (1111, 3000, 64), (2264, 4096, 128), (7700, 500, 64), (4800, 3200, 64)]
+          (1030, 256, 1536), (1111, 3000, 64), (2264, 4096, 128), (7700, 500, 64), (4800, 3200, 64), (700, 2360, 64),
+          (3136, 3072, 1024), (512, 1000, 2048), (300, 512, 2048), (352, 2048, 512), (384, 2048, 512)]
 
 
 def _data(M, N, K, dtype, gpu, n=1):
